@@ -633,6 +633,26 @@ int vtx_paged_decode_attention(const uint16_t* q, uint16_t* o, const uint16_t* k
                                int32_t num_kv_heads, int32_t group_size, int32_t head_dim,
                                int32_t page_size, float sm_scale, void* stream);
 
+/*
+ * vtx_paged_decode_attention for tables whose segments are few and long: a
+ * segment's pages may be split over several workgroups, whose partial results
+ * (fp32) a second launch on the stream combines.  workspace: scratch of at
+ * least vtx_paged_decode_attention_workspace_len floats, 16-byte aligned, its
+ * contents neither read nor kept across calls; where that length is 0 (no
+ * segment of such a table would be split) it may be NULL and the call is
+ * vtx_paged_decode_attention's.  How a segment is split depends on the
+ * table's contents alone, not on the buffers' capacity.
+ */
+int vtx_paged_decode_attention_split(const uint16_t* q, uint16_t* o, const uint16_t* k_cache,
+                                     const uint16_t* v_cache, int64_t cache_rows, const int32_t* kv_indptr,
+                                     const int32_t* kv_indices, int64_t kv_indices_len,
+                                     const int32_t* kv_last_page_len, int32_t batch_size,
+                                     int32_t num_kv_heads, int32_t group_size, int32_t head_dim,
+                                     int32_t page_size, float sm_scale, float* workspace,
+                                     int64_t workspace_len, void* stream);
+int64_t vtx_paged_decode_attention_workspace_len(int32_t batch_size, int32_t num_kv_heads, int32_t group_size,
+                                                 int32_t head_dim, int32_t page_size, int64_t kv_indices_len);
+
 /* 1 if vtx_paged_decode_attention handles this head_dim and group size. */
 int vtx_paged_decode_attention_supported(int32_t head_dim, int32_t group_size);
 

@@ -744,3 +744,54 @@ def test_sparse_attention_equals_dense_when_budget_covers_all(gpu):
     plan_decode(b.seq_lens, b.req_to_token, b.req_indices, ic)
     q, k, v = _attn_inputs(batch, gpu, 2, 128, 9)
     assert torch.equal(sparse_decode_attention(q, k, v, ic), dense_decode_attention(q, k, v, ic))
+
+
+# (request lengths, kv heads, page size, query heads per kv head, head dim):
+# one chunk more or less at the edges of a page and of a chunk, empty and short
+# requests beside long ones, many segments of uneven and of equal lengths
+_SPLIT_TABLES = {
+    "edge": ([2048, 2049, 2047], 1, 16, 2, 128),
+    "empty": ([0, 5000, 1, 700, 0], 2, 4, 1, 64),
+    "page1": ([3001], 2, 1, 4, 128),
+    "wide": ([1800, 33], 2, 32, 3, 256),
+    "heads8": ([6000, 16], 4, 64, 8, 128),
+    "uneven": ([9000, 300, 4100] + [1900 + 37 * i for i in range(15)], 8, 16, 2, 64),
+    "equal": ([2100] * 16, 8, 16, 2, 64),
+}
+
+
+@pytest.mark.parametrize("name", sorted(_SPLIT_TABLES))
+def test_decode_attention_split_segments(gpu, name):
+    """Tables whose segments are split over workgroups: within the bf16
+    rounding of the result of the oracle (fp32 sums over a few thousand
+    tokens add under 1e-5), the same bits whatever the buffer's capacity."""
+    from vortex_torch.decode_attention import paged_decode_attention
+    from vortex_torch.indexer.utils_sglang import plan_decode
+
+    lens, H, P, G, D = _SPLIT_TABLES[name]
+    pool = sum((n + P - 1) // P for n in lens) + 5
+    batch = W.make_batch(lens, pool_pages=pool, seed=41, page_size=P, num_kv_heads=H, group_size=G, head_dim=D)
+    ic, _ = W.make_contexts(batch, gpu)
+    b = batch.to(gpu)
+    plan_decode(b.seq_lens, b.req_to_token, b.req_indices, ic)
+    q, k, v = _attn_inputs(batch, gpu, G, D, 13)
+    ip, idx, last = ic.dense_kv_indptr, ic.dense_kv_indices, ic.kv_last_page_len
+    lib = _hip.load_library()
+    assert lib.vtx_paged_decode_attention_workspace_len(len(lens), H, G, D, P, idx.numel()) > 0
+    o = paged_decode_attention(q, k, v, ip, idx, last, len(lens), H)
+    exp = O.paged_decode_attention(_bits(q), _bits(k), _bits(v), _np(ip), _np(idx), _np(last), len(lens), H,
+                                   1.0 / np.sqrt(D))
+    np.testing.assert_allclose(_f(_bits(o)), _f(exp), rtol=2 ** -7, atol=1e-4)
+    more = torch.cat([idx, torch.full((3 * idx.numel(),), -7, dtype=torch.int32, device=gpu)])
+    assert torch.equal(paged_decode_attention(q, k, v, ip, more, last, len(lens), H), o)
+    # entries outside the pool are left out, as without the split
+    bad = idx.clone()
+    bad[::5] = -1
+    bad[1::9] = pool * H
+    got = paged_decode_attention(q, k, v, ip, bad, last, len(lens), H)
+    whole = torch.empty_like(q)
+    rc = lib.vtx_paged_decode_attention(q.data_ptr(), whole.data_ptr(), k.data_ptr(), v.data_ptr(), k.shape[0],
+                                        ip.data_ptr(), bad.data_ptr(), bad.numel(), last.data_ptr(), len(lens), H, G,
+                                        D, P, 1.0 / np.sqrt(D), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    np.testing.assert_allclose(_f(_bits(got)), _f(_bits(whole)), rtol=2 ** -7, atol=1e-4)

@@ -10,7 +10,9 @@
 // with fp32 scores, an fp32 online softmax and fp32 accumulation.  A segment
 // with no tokens writes zeros.
 //
-// One workgroup per segment (8 waves, or 4 for wide G x D).  The segment's
+// One workgroup per segment, or per chunk of a segment where segments are few
+// and long (the chunks' partial outputs then combined by a second launch);
+// 8 waves, or 4 for wide G x D.  The segment's
 // page rows are staged in LDS first (one load per page, up to kPageCap
 // pages; longer segments read them from the table), so each batch of a
 // wave costs one memory round trip: a wave takes every kWaves-th batch of
@@ -40,8 +42,78 @@ struct AttnArgs {
   int64_t indices_len;
   const int32_t* last_len;
   int32_t segments, G, D, P;
+  int32_t p_shift;  // log2(P), or -1
   float scale;
+  // split segments (vtx_paged_decode_attention_split): up to nsplit chunks
+  // per segment (chunks_of); ml and acc hold a chunk's (max, sum) and
+  // unnormalised output, [segments, nsplit, G(, D)]
+  int32_t nsplit, cus, min_avg_tokens;
+  int32_t ragged_only;  // split only tables of uneven segments
+  float2* ml;
+  float* acc;
 };
+
+constexpr int kMaxSplit = 128;             // chunks per segment
+constexpr int kMaxSplitSegmentsPerCu = 4;  // from so many segments per CU on nothing is split
+constexpr int kMinChunkTokens = 128;
+constexpr int kFewChunkTokens = 256;
+
+// Chunks of a segment of m pages (1: not split) and the pages of each, from
+// the table's total page count: a function of the table alone (the same in
+// the attention and the combine kernel, and for two tables that hold the same
+// pages in buffers of different capacity).
+//
+// A table is split when its segments hold min_avg_tokens on average and,
+// with half a segment per CU and more, the longest is over 1.3 times the
+// average (split_plan says why).  A workgroup takes about 5.5 us + 12.6 us per
+// 1024 tokens (its dot products, not its loads, set that; 1024 threads took as
+// long) until all of them together reach the card's read rate, the combine
+// launch 2.5 us.  So a few short segments want one chunk of 128-256 tokens per
+// CU (8 segments of 2048 tokens: 11.4 us with chunks of 128, 13.1 with 256; 64
+// segments of 1024: 19.0 and 16.0), and long ones four chunks per CU in all,
+// which even out ragged lengths without making the chunks short (128 segments
+// of 1k to 16k tokens: 107 us, 112 with two or eight and 137 with sixteen).
+struct Chunks {
+  uint32_t count, pages;
+};
+__device__ __forceinline__ Chunks chunks_of(const AttnArgs& a, uint32_t m, uint32_t longest, int32_t first,
+                                            int32_t end) {
+  const long long all = (long long)end - first;
+  const uint32_t total = all < 0 ? 0u : (uint32_t)(all < a.indices_len ? all : a.indices_len);
+  Chunks c{1u, m};
+  if (m == 0 || (unsigned long long)total * a.P < (unsigned long long)a.min_avg_tokens * a.segments) return c;
+  if (a.ragged_only && 10ull * longest * a.segments <= 13ull * total) return c;
+  const uint32_t least = (kMinChunkTokens + a.P - 1) / a.P, few = (kFewChunkTokens + a.P - 1) / a.P;
+  uint32_t per = total / a.cus;
+  per = per < least ? least : (per > few ? few : per);
+  const uint32_t even = (total + 4 * a.cus - 1) / (4 * a.cus);
+  per = per < even ? even : per;
+  uint32_t n = (m + per - 1) / per;
+  n = n > (uint32_t)a.nsplit ? (uint32_t)a.nsplit : n;
+  c.pages = (m + n - 1) / n;
+  c.count = (m + c.pages - 1) / c.pages;
+  return c;
+}
+
+// Pages of the table's longest segment (0 where chunks_of does not ask).  Every
+// thread of the workgroup calls it; red: LDS, one entry per wave, free again
+// after the caller's next barrier.
+template <int T>
+__device__ __forceinline__ uint32_t longest_segment(const AttnArgs& a, uint32_t* red) {
+  if (!a.ragged_only) return 0;  // uniform
+  uint32_t mx = 0;
+  for (int i = threadIdx.x; i < a.segments; i += T) {
+    const int32_t d = (int32_t)((uint32_t)a.indptr[i + 1] - (uint32_t)a.indptr[i]);
+    mx = d > 0 && (uint32_t)d > mx ? (uint32_t)d : mx;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) mx = max(mx, vtx::xshfl(mx, d));
+  if (vtx::lane_id() == 0) red[threadIdx.x / vtx::kWave] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < T / vtx::kWave; ++w) mx = max(mx, red[w]);
+  return mx;
+}
 
 // Threads per workgroup: 8 waves where a wave's registers fit 128 (rows of
 // one 16-byte vector per lane, at most two query heads), else 4.
@@ -56,7 +128,7 @@ constexpr int attn_batch() {
 }
 
 // With 8 waves, at most 128 registers (four waves per SIMD: two workgroups per CU).
-template <int LPR, int VPL, int kG>
+template <int LPR, int VPL, int kG, bool kSplit>
 __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
                              (attn_threads<LPR, VPL, kG>() == 512 ? 4 : 1)) void paged_decode_attention_kernel(AttnArgs a) {
   constexpr int T = attn_threads<LPR, VPL, kG>();
@@ -64,11 +136,13 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
   constexpr int kRowsPerLoad = vtx::kWave / LPR;  // tokens per wave-wide load
   constexpr int kB = attn_batch<VPL, kG>();        // token groups per batch
   __shared__ int32_t s_rows[kPageCap];
+  __shared__ uint32_t s_red[kWaves];
   __shared__ float s_m[kWaves][kG];
   __shared__ float s_l[kWaves][kG];
   __shared__ float s_acc[kWaves][kG][LPR * VPL * 8];
 
-  const int seg = blockIdx.x;
+  const int seg = kSplit ? (int)(blockIdx.x % (uint32_t)a.segments) : (int)blockIdx.x;
+  const int chunk = kSplit ? (int)(blockIdx.x / (uint32_t)a.segments) : 0;
   const int tid = threadIdx.x;
   const int wave = vtx::uniform(tid / vtx::kWave);
   const int lane = vtx::lane_id();
@@ -76,14 +150,31 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
   const int col = lane % LPR;
   const int G = a.G, D = a.D, P = a.P;
 
-  const long long start = a.indptr[seg];
-  const long long m = (long long)a.indptr[seg + 1] - start;
-  int T_tok = 0;  // tokens of the segment
+  long long start = a.indptr[seg];
+  long long m = (long long)a.indptr[seg + 1] - start;
+  int T_tok = 0;  // tokens of the segment (of the chunk)
+  int nchunks = 1;
   if (m > 0 && start >= 0 && start + m <= a.indices_len && a.rows > 0) {
     int last = a.last_len[seg];
     last = last < 0 ? 0 : (last > P ? P : last);
     const long long t = (m - 1) * P + last;
     T_tok = t < (1LL << 30) ? (int)t : 0;  // (token indices, with the prefetch past the end, fit an int)
+    if constexpr (kSplit) {
+      if (T_tok > 0) {
+        const Chunks c = chunks_of(a, (uint32_t)m, longest_segment<T>(a, s_red), a.indptr[0], a.indptr[a.segments]);
+        nchunks = (int)c.count;
+        if (chunk < nchunks) {  // this chunk's pages as a segment of their own
+          const int p0 = chunk * (int)c.pages;
+          const int p1 = min((int)m, p0 + (int)c.pages);
+          T_tok = (p1 == (int)m ? T_tok : p1 * P) - p0 * P;
+          start += p0;
+          m = p1 - p0;
+        }
+      }
+    }
+  }
+  if constexpr (kSplit) {
+    if (chunk >= nchunks) return;  // uniform
   }
   // query slice of this lane (columns (v * LPR + col) * 8 .. + 8), requested
   // first so that it arrives with the page rows; heads past G read head
@@ -142,7 +233,7 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
       const int t = ((wave + kWaves * j) * kB + i) * kRowsPerLoad + grp;
       int row = -1, slot = 0;
       if (t < T_tok) {
-        const int pg = t / P;
+        const int pg = a.p_shift >= 0 ? t >> a.p_shift : t / P;
         slot = t - pg * P;
         if (staged) {
           row = s_rows[pg];
@@ -258,13 +349,107 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
         O = fmaf(s_acc[w][g][d], f, O);
       }
     }
+    if constexpr (kSplit) {
+      if (nchunks > 1) {  // uniform: for the combine kernel
+        const long long row = ((long long)seg * a.nsplit + chunk) * G + g;
+        a.acc[row * D + d] = O;
+        if (d == 0) a.ml[row] = float2{M, L};
+        continue;
+      }
+    }
     a.o[((long long)seg * G + g) * D + d] = (uint16_t)vtx::f32_to_bf16(L > 0.f ? O / L : 0.f);
+  }
+}
+
+// Outputs of the split segments: one workgroup per (segment, query head)
+// weighs its chunks' partial outputs, wave w those of chunks w, w + kCombineWaves,
+// ... (lane l of the wave holds the (max, sum) of the l-th of them); the waves'
+// (max, sum, output) are merged in LDS.
+constexpr int kCombineWaves = 4;
+static_assert(kMaxSplit <= kCombineWaves * vtx::kWave, "one lane per chunk");
+template <int kD>
+__global__ __launch_bounds__(kCombineWaves * vtx::kWave) void attention_combine_kernel(AttnArgs a) {
+  constexpr int kCols = kD / vtx::kWave;
+  constexpr int kAhead = 8;  // chunks loaded before any is added
+  __shared__ uint32_t s_red[kCombineWaves];
+  __shared__ float s_m[kCombineWaves];
+  __shared__ float s_l[kCombineWaves];
+  __shared__ float s_o[kCombineWaves][kD];
+  const long long row = blockIdx.x;
+  const int seg = (int)(row / a.G);
+  const int g = (int)(row % a.G);
+  const int wave = vtx::uniform(threadIdx.x / vtx::kWave);
+  const int lane = vtx::lane_id();
+  const long long start = a.indptr[seg];
+  const long long m = (long long)a.indptr[seg + 1] - start;
+  const int32_t last = a.last_len[seg];
+  if (!(m > 0 && start >= 0 && start + m <= a.indices_len && a.rows > 0)) return;  // uniform, as the returns below
+  const long long tok = (m - 1) * a.P + (last < 0 ? 0 : (last > a.P ? a.P : last));
+  if (tok <= 0 || tok >= (1LL << 30)) return;
+  const uint32_t longest = longest_segment<kCombineWaves * vtx::kWave>(a, s_red);
+  const int all = (int)chunks_of(a, (uint32_t)m, longest, a.indptr[0], a.indptr[a.segments]).count;
+  if (all <= 1) return;  // written by its workgroup
+  // this wave's chunks (none: wave 0's first again, with weight 0)
+  const int n = all > wave ? (all - wave + kCombineWaves - 1) / kCombineWaves : 0;
+  auto at = [&](int i) {  // row of the i-th of them in ml and acc
+    const int c = i < n ? wave + kCombineWaves * i : 0;
+    return ((long long)seg * a.nsplit + c) * a.G + g;
+  };
+  const float2 ml = a.ml[at(lane)];
+  float M = lane < n ? ml.x : -INFINITY;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) M = fmaxf(M, vtx::xshfl(M, d));
+  const float w = lane < n && M != -INFINITY ? __expf(ml.x - M) : 0.f;
+  const float L = vtx::wave_sum(w * ml.y);
+  float O[kCols];
+#pragma unroll
+  for (int j = 0; j < kCols; ++j) O[j] = 0.f;
+  for (int i0 = 0; i0 < n; i0 += kAhead) {
+    float v[kAhead][kCols];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+      for (int j = 0; j < kCols; ++j) v[i][j] = a.acc[at(i0 + i) * kD + j * vtx::kWave + lane];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const float f = i0 + i < n ? __uint_as_float(vtx::lane_value(__float_as_uint(w), i0 + i)) : 0.f;
+#pragma unroll
+      for (int j = 0; j < kCols; ++j) O[j] = i0 + i < n ? fmaf(v[i][j], f, O[j]) : O[j];
+    }
+  }
+  if (lane == 0) {
+    s_m[wave] = M;
+    s_l[wave] = L;
+  }
+#pragma unroll
+  for (int j = 0; j < kCols; ++j) s_o[wave][j * vtx::kWave + lane] = O[j];
+  __syncthreads();
+  for (int d = threadIdx.x; d < kD; d += kCombineWaves * vtx::kWave) {
+    float MM = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < kCombineWaves; ++v) MM = fmaxf(MM, s_m[v]);
+    float LL = 0.f, OO = 0.f;
+    if (MM != -INFINITY) {
+#pragma unroll
+      for (int v = 0; v < kCombineWaves; ++v) {
+        const float f = __expf(s_m[v] - MM);
+        LL = fmaf(s_l[v], f, LL);
+        OO = fmaf(s_o[v][d], f, OO);
+      }
+    }
+    a.o[row * kD + d] = (uint16_t)vtx::f32_to_bf16(LL > 0.f ? OO / LL : 0.f);
   }
 }
 
 template <int LPR, int VPL, int kG>
 void launch_one(const AttnArgs& a, hipStream_t s) {
-  paged_decode_attention_kernel<LPR, VPL, kG><<<a.segments, attn_threads<LPR, VPL, kG>(), 0, s>>>(a);
+  constexpr int T = attn_threads<LPR, VPL, kG>();
+  if (a.nsplit == 1) {
+    paged_decode_attention_kernel<LPR, VPL, kG, false><<<a.segments, T, 0, s>>>(a);
+    return;
+  }
+  paged_decode_attention_kernel<LPR, VPL, kG, true><<<a.segments * a.nsplit, T, 0, s>>>(a);
+  attention_combine_kernel<LPR * VPL * 8><<<a.segments * a.G, kCombineWaves * vtx::kWave, 0, s>>>(a);
 }
 
 template <int LPR, int VPL>
@@ -282,14 +467,42 @@ extern "C" int vtx_paged_decode_attention_supported(int32_t head_dim, int32_t gr
   return (head_dim == 64 || head_dim == 128 || head_dim == 256) && group_size >= 1 && group_size <= 8;
 }
 
-extern "C" int vtx_paged_decode_attention(const uint16_t* q, uint16_t* o, const uint16_t* k_cache,
-                                          const uint16_t* v_cache, int64_t cache_rows, const int32_t* kv_indptr,
-                                          const int32_t* kv_indices, int64_t kv_indices_len,
-                                          const int32_t* kv_last_page_len, int32_t batch_size,
-                                          int32_t num_kv_heads, int32_t group_size, int32_t head_dim,
-                                          int32_t page_size, float sm_scale, void* stream) {
-  vtx::clear_error();
-  const char* what = "paged_decode_attention";
+namespace {
+
+// How a call may split its segments: up to nsplit chunks each (1: not at
+// all), in tables whose segments hold min_avg_tokens on average.
+struct SplitPlan {
+  int32_t nsplit, cus, min_avg_tokens, ragged_only;
+};
+
+// Fewer than half a segment per CU leave the chip idle, so splitting pays
+// from about 500 tokens on (8 segments: 512 tokens 11.5 -> 10.7 us, 2048
+// tokens 31.4 -> 11.4; 64 segments: 768 tokens 15.2 -> 14.7, 1024 tokens
+// 19.2 -> 16.5; the line 384 + 8 tokens per segment keeps 32 segments of 512,
+// 11.8 against 12.7, whole).  With more segments a table gains by evening out
+// its lengths (128 segments of 1k to 16k tokens: 219 -> 108 us; 256 of 0.5k to
+// 8k: 128 -> 109), and one of equal lengths only pays for the combine launch
+// (128 of 2048: 32.3 us, 34.2 with it; 256: 46.6 and 48.8), so from a segment
+// per CU on, where an uneven table gains least, the line lies at 4096.
+SplitPlan split_plan(long long segments, long long indices_len, int32_t page_size) {
+  const int cus = vtx::device_cu_count();
+  SplitPlan p{1, 1, 0, 0};
+  if (cus <= 0 || segments <= 0 || segments >= kMaxSplitSegmentsPerCu * (long long)cus) return p;
+  p.cus = cus;
+  p.ragged_only = 2 * segments >= cus;
+  p.min_avg_tokens = !p.ragged_only ? (int32_t)(384 + 8 * segments) : (segments < cus ? 2048 : 4096);
+  // (a table that cannot hold this average is not split whatever it holds)
+  if (indices_len * page_size < (long long)p.min_avg_tokens * segments) return p;
+  const long long n = (8LL * cus + segments - 1) / segments;
+  p.nsplit = (int32_t)(n > kMaxSplit ? kMaxSplit : n);
+  return p;
+}
+
+int attention_impl(const char* what, const uint16_t* q, uint16_t* o, const uint16_t* k_cache,
+                   const uint16_t* v_cache, int64_t cache_rows, const int32_t* kv_indptr, const int32_t* kv_indices,
+                   int64_t kv_indices_len, const int32_t* kv_last_page_len, int32_t batch_size, int32_t num_kv_heads,
+                   int32_t group_size, int32_t head_dim, int32_t page_size, float sm_scale, float* workspace,
+                   int64_t workspace_len, void* stream) {
   if (batch_size < 0 || num_kv_heads < 1 || page_size < 1 || cache_rows < 0 || kv_indices_len < 0)
     return vtx::fail(VTX_E_INVALID, "%s: bad sizes", what);
   if (!vtx_paged_decode_attention_supported(head_dim, group_size))
@@ -316,11 +529,71 @@ extern "C" int vtx_paged_decode_attention(const uint16_t* q, uint16_t* o, const 
   a.G = group_size;
   a.D = head_dim;
   a.P = page_size;
+  a.p_shift = vtx::log2_exact(page_size);
   a.scale = sm_scale;
+  a.nsplit = 1;
+  a.cus = 1;
+  a.min_avg_tokens = 0;
+  a.ragged_only = 0;
+  a.ml = nullptr;
+  a.acc = nullptr;
+  if (workspace) {
+    const SplitPlan p = split_plan(segments, kv_indices_len, page_size);
+    const long long rows = segments * p.nsplit * group_size;
+    if (p.nsplit > 1) {
+      if (workspace_len < rows * (head_dim + 2) || !vtx::aligned16(workspace))
+        return vtx::fail(VTX_E_INVALID, "%s: workspace of %lld floats (16-byte aligned) needed, got %lld", what,
+                         rows * (long long)(head_dim + 2), (long long)workspace_len);
+      a.nsplit = p.nsplit;
+      a.cus = p.cus;
+      a.min_avg_tokens = p.min_avg_tokens;
+      a.ragged_only = p.ragged_only;
+      a.acc = workspace;
+      a.ml = reinterpret_cast<float2*>(workspace + rows * head_dim);
+    }
+  }
   hipStream_t s = vtx::as_stream(stream);
   switch (head_dim) {
     case 64: return launch_g<8, 1>(a, s);
     case 128: return launch_g<16, 1>(a, s);
     default: return launch_g<16, 2>(a, s);
   }
+}
+
+}  // namespace
+
+extern "C" int vtx_paged_decode_attention(const uint16_t* q, uint16_t* o, const uint16_t* k_cache,
+                                          const uint16_t* v_cache, int64_t cache_rows, const int32_t* kv_indptr,
+                                          const int32_t* kv_indices, int64_t kv_indices_len,
+                                          const int32_t* kv_last_page_len, int32_t batch_size,
+                                          int32_t num_kv_heads, int32_t group_size, int32_t head_dim,
+                                          int32_t page_size, float sm_scale, void* stream) {
+  vtx::clear_error();
+  return attention_impl("paged_decode_attention", q, o, k_cache, v_cache, cache_rows, kv_indptr, kv_indices,
+                        kv_indices_len, kv_last_page_len, batch_size, num_kv_heads, group_size, head_dim, page_size,
+                        sm_scale, nullptr, 0, stream);
+}
+
+extern "C" int64_t vtx_paged_decode_attention_workspace_len(int32_t batch_size, int32_t num_kv_heads,
+                                                            int32_t group_size, int32_t head_dim, int32_t page_size,
+                                                            int64_t kv_indices_len) {
+  if (batch_size < 0 || num_kv_heads < 1 || page_size < 1 || kv_indices_len < 0 ||
+      !vtx_paged_decode_attention_supported(head_dim, group_size))
+    return 0;
+  const long long segments = (long long)batch_size * num_kv_heads;
+  const SplitPlan p = split_plan(segments, kv_indices_len, page_size);
+  return p.nsplit > 1 ? segments * p.nsplit * group_size * (head_dim + 2) : 0;
+}
+
+extern "C" int vtx_paged_decode_attention_split(const uint16_t* q, uint16_t* o, const uint16_t* k_cache,
+                                                const uint16_t* v_cache, int64_t cache_rows,
+                                                const int32_t* kv_indptr, const int32_t* kv_indices,
+                                                int64_t kv_indices_len, const int32_t* kv_last_page_len,
+                                                int32_t batch_size, int32_t num_kv_heads, int32_t group_size,
+                                                int32_t head_dim, int32_t page_size, float sm_scale,
+                                                float* workspace, int64_t workspace_len, void* stream) {
+  vtx::clear_error();
+  return attention_impl("paged_decode_attention", q, o, k_cache, v_cache, cache_rows, kv_indptr, kv_indices,
+                        kv_indices_len, kv_last_page_len, batch_size, num_kv_heads, group_size, head_dim, page_size,
+                        sm_scale, workspace, workspace_len, stream);
 }

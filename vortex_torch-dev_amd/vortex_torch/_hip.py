@@ -121,6 +121,11 @@ _SIGNATURES = {
         [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i32, _i32, _i32, _i32, _i32, ctypes.c_float, _vp],
         ctypes.c_int,
     ),
+    "vtx_paged_decode_attention_split": (
+        [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i32, _i32, _i32, _i32, _i32, ctypes.c_float, _vp, _i64, _vp],
+        ctypes.c_int,
+    ),
+    "vtx_paged_decode_attention_workspace_len": ([_i32, _i32, _i32, _i32, _i32, _i64], ctypes.c_int64),
     "vtx_paged_decode_attention_supported": ([_i32, _i32], ctypes.c_int),
     "vtx_bf16_rounding_check": ([_vp, _vp], ctypes.c_int),
     "vtx_stream_capture_id": ([_vp, ctypes.POINTER(ctypes.c_ulonglong)], ctypes.c_int),
@@ -1018,9 +1023,13 @@ def paged_decode_attention(q, o, k_cache, v_cache, kv_indptr, kv_indices, kv_las
     if kv_indptr.numel() < B * H + 1 or kv_last_page_len.numel() < B * H:
         raise RuntimeError(f"vortex_torch: kv_indptr needs {B * H + 1} and kv_last_page_len {B * H} entries")
     with _on_device(dev):
-        rc = lib.vtx_paged_decode_attention(q.data_ptr(), o.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), rows,
-                                            kv_indptr.data_ptr(), kv_indices.data_ptr(), kv_indices.numel(),
-                                            kv_last_page_len.data_ptr(), B, H, G, D, P, float(sm_scale), _stream(dev))
+        n = lib.vtx_paged_decode_attention_workspace_len(B, H, G, D, P, kv_indices.numel())
+        # the chunks' partial results, on the current stream (which both launches run on)
+        ws = torch.empty(n, dtype=torch.float32, device=dev) if n > 0 else None
+        rc = lib.vtx_paged_decode_attention_split(
+            q.data_ptr(), o.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), rows, kv_indptr.data_ptr(),
+            kv_indices.data_ptr(), kv_indices.numel(), kv_last_page_len.data_ptr(), B, H, G, D, P, float(sm_scale),
+            None if ws is None else ws.data_ptr(), n, _stream(dev))
     _check(rc, "paged_decode_attention")
 
 
