@@ -150,15 +150,17 @@ DECODE_CONFIGS = {
 
 
 def fused_kernel_name(batch: W.DecodeBatch) -> str:
-    """Kernel instance the fused launch selects (VTX_FUSED_AUTO: split layout
-    when there are fewer than two segments per compute unit)."""
+    """Kernel instance the fused launch selects (VTX_FUSED_AUTO: the library's
+    split_pays and segment_threads)."""
     from vortex_torch._deferred import fused_layout
 
     lpr, vpl = {64: (8, 1), 128: (16, 1), 256: (16, 2), 512: (16, 4), 576: (8, 9)}[batch.head_dim]
     segments = batch.batch * batch.num_kv_heads
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     layout = fused_layout()
-    if layout == 2 or (layout == 0 and segments < 2 * cus):
+    mp = batch.max_pages_per_request
+    auto = segments < 2 * cus if batch.head_dim >= 256 else mp > 512 and 3 * segments < 2 * cus
+    if layout == 2 or (layout == 0 and auto):
         # the library's split_threads / split_pass / chunk choice, with the
         # topK op's workspace (staging zone present)
         D = batch.head_dim
@@ -176,8 +178,7 @@ def fused_kernel_name(batch: W.DecodeBatch) -> str:
         else:
             T, kpass = (512 if D <= 256 else 256), small_pass * (2 if large else 1)
         return f"indexer_split_kernel<{T}, {lpr}, {vpl}, {kpass}, {cm}>"
-    mp = batch.max_pages_per_request
-    T = 256 if mp <= 256 else (512 if mp <= 1024 else 1024)
+    T = 256 if mp <= 256 else (512 if mp <= 512 or batch.head_dim >= 512 or segments > cus else 1024)
     # the decode CMean (loc: one token per request) runs in the same launch
     # for rows of one vector per lane, with loc in one register per lane up
     # to 64 tokens, four up to 256

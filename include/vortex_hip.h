@@ -213,8 +213,10 @@ int vtx_topk_select(const uint16_t* score, int64_t score_len,
  * first call, and every call that completes leaves it all zero.
  * A shorter buffer (at least eff_batch_size entries) holds counters only.
  * Calls that share one workspace must be ordered on one stream.  mode: VTX_FUSED_AUTO
- * (split when there are fewer than two segments per compute unit and the
- * counters are given), VTX_FUSED_SEGMENT or VTX_FUSED_SPLIT.  Outputs are
+ * (with the counters given, split where few segments would leave compute units
+ * idle for longer than a split segment's hand-off takes: head_dim >= 256 and
+ * fewer than two segments per compute unit, or head_dim <= 128, over 512 pages
+ * and fewer than two for three units), VTX_FUSED_SEGMENT or VTX_FUSED_SPLIT.  Outputs are
  * identical in every mode.
  *
  * schedule (optional, NULL for none): the fused_schedule vtx_plan_decode

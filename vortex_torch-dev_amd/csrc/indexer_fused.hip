@@ -1243,6 +1243,34 @@ int split_chunk(int dim, bool large, bool quad) {
   return (split_threads(dim, large, quad) / 64) * split_pass(dim, large, quad);
 }
 
+// Whether AUTO takes the split layout, for segments of at most max_pages
+// pages.  Fewer than two segments per CU leave CUs idle with one workgroup
+// per segment, but a split segment's hand-off (two device-scope round trips
+// and a merge) takes longer than a second pass of rows: it pays for wide rows
+// (D >= 256; 8 MLA segments of 256 pages 9.7 us per layer against 19), and at
+// D <= 128 for segments of several passes (over 512 pages) that leave a third
+// of the CUs idle.  Measured per layer, segment / split: 8 segments of 256
+// pages 7.0 / 9.0 us, 64 of 512 10.3 / 10.6 (top-64), 256 of 512 9.8 / 11.9,
+// 256 of 1024 15.0 / 17.1, 256 of 2048 25.0 / 28.2; 8 of 1024 pages 12.2 /
+// 9.8, 64 of 1024 12.4 / 10.7, 128 of 1024 12.9 / 12.2, 64 of 2048 24 / 14.
+bool split_pays(long long segments, long long max_pages, int dim, int cus) {
+  if (dim >= 256) return segments < 2LL * cus;
+  return max_pages > 512 && 3 * segments < 2LL * cus;
+}
+
+// Threads per workgroup of the segment layout: every page of a segment in one
+// pass where the pages allow it (4, 8 or 16 waves of 64), and past 512 pages
+// 16 waves only where each CU has at most one workgroup.  Two workgroups of 8
+// waves per CU do one's select while the other's rows arrive (512 segments of
+// up to 2048 pages: 33.0 us per layer, 37.9 with 16 waves); alone on a CU, 16
+// waves are faster (256 segments of up to 1024 pages: 14.9 us, 16.6 with 8).
+// Rows of four or more vectors per lane need more than the 128 registers a
+// lane of a 1024-thread workgroup can have.
+int segment_threads(long long segments, long long max_pages, int dim, int cus) {
+  if (max_pages <= 256) return 256;
+  return max_pages <= 512 || dim >= 512 || segments > cus ? 512 : 1024;
+}
+
 // blocks: the grid, xcd: work ids per XCD (8 * xcd workgroups take work
 // ids, the rest are CMean tile workgroups)
 template <int P, int kCm>
@@ -1448,11 +1476,8 @@ int fused_impl(const uint16_t* q, int64_t q_rows, int32_t group_size, const uint
   const int cus = vtx::device_cu_count();
   if (cus <= 0) return vtx::fail(VTX_E_DEVICE, "indexer_fused: cannot query the compute unit count");
 
-  // One workgroup per segment fills the chip when there are at least two
-  // segments per CU; fewer (long contexts, MLA's single latent head) leave
-  // CUs idle, so their pages are split over several workgroups.
   const bool split = mode == VTX_FUSED_SPLIT ||
-                     (mode == VTX_FUSED_AUTO && have_counters && (long long)eff_batch_size < 2LL * cus);
+                     (mode == VTX_FUSED_AUTO && have_counters && split_pays(eff_batch_size, want, head_dim, cus));
   // The CMean runs inside the launch for decode-sized loc and a 16-byte
   // aligned K pool: in the segment layout for rows of one 16-byte vector per
   // lane (its tile layout is then the scoring layout), in the split layout
@@ -1547,11 +1572,11 @@ int fused_impl(const uint16_t* q, int64_t q_rows, int32_t group_size, const uint
   if (grid > 0x7fffffffLL) return vtx::fail(VTX_E_INVALID, "indexer_fused: too many query rows");
   const long long blocks = grid;
   if (blocks == 0) return VTX_OK;
-  if (max_num_pages <= 256) return launch_dim<256>(a, cmp, (int)blocks, lds, s);
-  // (rows of four or more vectors per lane need more than the 128 registers
-  // a lane of a 1024-thread workgroup can have)
-  if (max_num_pages <= 1024 || head_dim >= 512) return launch_dim<512>(a, cmp, (int)blocks, lds, s);
-  return launch_dim<1024>(a, cmp, (int)blocks, lds, s);
+  switch (segment_threads(eff_batch_size, want, head_dim, cus)) {
+    case 256: return launch_dim<256>(a, cmp, (int)blocks, lds, s);
+    case 512: return launch_dim<512>(a, cmp, (int)blocks, lds, s);
+    default: return launch_dim<1024>(a, cmp, (int)blocks, lds, s);
+  }
 }
 
 }  // namespace
