@@ -464,6 +464,32 @@ def test_quest_fused_equals_unfused(gpu, monkeypatch, name):
         assert (out["0"][4].reshape(-1, G * batch.head_dim)[cov] != sentinel).any()
 
 
+@pytest.mark.parametrize("flow_name", ["gqa_quest_sparse_attention", "gqa_block_sparse_attention"])
+@pytest.mark.parametrize("pages,requests", [([67, 250, 256, 33], 4), ([512, 511, 81, 34, 497], 5),
+                                            ([1030, 513, 1024, 70], 4), ([1030, 513, 97, 50], 130)])
+@pytest.mark.parametrize("G,D", [(1, 128), (2, 64), (2, 128), (3, 128)])
+def test_flow_fused_equals_unfused_at_share_edges(gpu, monkeypatch, flow_name, pages, requests, G, D):
+    """Page counts at the edges of a wave's share and of the steps it goes
+    through, for every workgroup size (260 segments: over one per compute unit
+    of 256), the closed last pages scored (eos 0): the fused launch writes
+    what the separate launches write."""
+    lens = [2 * n for n in pages] + [2 * (33 + i % 40) - i % 2 for i in range(requests - len(pages))]
+    batch = W.make_batch(lens, pool_pages=sum((n + 1) // 2 for n in lens) + 3, seed=61, page_size=2, num_kv_heads=2,
+                         group_size=G, head_dim=D, topk=30, eos=0)
+    out = {}
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("VORTEX_FUSE", fuse)
+        run = _Flow(flow_name, batch, gpu)
+        run.flow.max_op.output_buffer.zero_()
+        run.ic.sparse_kv_indices.fill_(-1)
+        run.step()
+        torch.cuda.synchronize()
+        out[fuse] = [_np(run.ic.sparse_kv_indices), _bits(run.flow.max_op.output_buffer)]
+        out[fuse] += [_bits(t) for n, t in sorted(run.cache.items()) if n not in ("k", "v")]
+    for a, b in zip(out["1"], out["0"]):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_quest_fused_keeps_observed_intermediates(gpu, monkeypatch):
     """An intermediate still referenced after forward_indexer is computed."""
     batch = W.c1()

@@ -1258,19 +1258,6 @@ bool split_pays(long long segments, long long max_pages, int dim, int cus) {
   return max_pages > 512 && 3 * segments < 2LL * cus;
 }
 
-// Threads per workgroup of the segment layout: every page of a segment in one
-// pass where the pages allow it (4, 8 or 16 waves of 64), and past 512 pages
-// 16 waves only where each CU has at most one workgroup.  Two workgroups of 8
-// waves per CU do one's select while the other's rows arrive (512 segments of
-// up to 2048 pages: 33.0 us per layer, 37.9 with 16 waves); alone on a CU, 16
-// waves are faster (256 segments of up to 1024 pages: 14.9 us, 16.6 with 8).
-// Rows of four or more vectors per lane need more than the 128 registers a
-// lane of a 1024-thread workgroup can have.
-int segment_threads(long long segments, long long max_pages, int dim, int cus) {
-  if (max_pages <= 256) return 256;
-  return max_pages <= 512 || dim >= 512 || segments > cus ? 512 : 1024;
-}
-
 // blocks: the grid, xcd: work ids per XCD (8 * xcd workgroups take work
 // ids, the rest are CMean tile workgroups)
 template <int P, int kCm>
@@ -1572,7 +1559,10 @@ int fused_impl(const uint16_t* q, int64_t q_rows, int32_t group_size, const uint
   if (grid > 0x7fffffffLL) return vtx::fail(VTX_E_INVALID, "indexer_fused: too many query rows");
   const long long blocks = grid;
   if (blocks == 0) return VTX_OK;
-  switch (segment_threads(eff_batch_size, want, head_dim, cus)) {
+  // (rows of four or more vectors per lane need more than the 128 registers
+  // a lane of a 1024-thread workgroup can have)
+  const int threads = vtx::segment_threads(eff_batch_size, want, cus);
+  switch (head_dim >= 512 && threads > 512 ? 512 : threads) {
     case 256: return launch_dim<256>(a, cmp, (int)blocks, lds, s);
     case 512: return launch_dim<512>(a, cmp, (int)blocks, lds, s);
     default: return launch_dim<1024>(a, cmp, (int)blocks, lds, s);

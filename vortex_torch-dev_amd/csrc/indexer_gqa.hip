@@ -483,9 +483,11 @@ int gqa_impl(const uint16_t* q, int64_t q_rows, int32_t group_size, const uint16
     cma.page_shift = vtx::log2_exact(cms->page_size);
   }
   const vtx::CmArgs* cmp = cm_launch ? &cma : nullptr;
-  if (max_num_pages <= 256) return launch_g<256>(a, cmp, eff_batch_size, lds, s);
-  if (max_num_pages <= 1024) return launch_g<512>(a, cmp, eff_batch_size, lds, s);
-  return launch_g<1024>(a, cmp, eff_batch_size, lds, s);
+  switch (vtx::segment_threads(eff_batch_size, max_num_pages, vtx::device_cu_count())) {
+    case 256: return launch_g<256>(a, cmp, eff_batch_size, lds, s);
+    case 512: return launch_g<512>(a, cmp, eff_batch_size, lds, s);
+    default: return launch_g<1024>(a, cmp, eff_batch_size, lds, s);
+  }
 }
 
 }  // namespace

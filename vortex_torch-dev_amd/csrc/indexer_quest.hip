@@ -46,12 +46,7 @@ struct QuestArgs {
 // the xor tree over the LPR lanes, as quest_pass_multi computes it.
 template <int LPR>
 __device__ __forceinline__ float quest_vec(const vtx::U4& mx, const vtx::U4& mn, const float (&xs)[8]) {
-  float a[8], b[8];
-  vtx::unpack8(mx, a);
-  vtx::unpack8(mn, b);
-  float s = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) s += vtx::bf16r(fmaxf(xs[e] * a[e], xs[e] * b[e]));
+  float s = vtx::quest_add(mx, mn, xs, 0.f);
 #pragma unroll
   for (int d = LPR / 2; d >= 1; d >>= 1) s += vtx::xshfl(s, d);
   return s;
@@ -78,11 +73,20 @@ __global__ __launch_bounds__(T, (VPL == 1 ? 4 : (VPL <= 4 ? 2 : 1))) void quest_
   constexpr int kPass = (VPL == 1 && kCmRegs == 0) ? 32 : 16;
   constexpr bool cm_on = kCmRegs > 0 && VPL == 1;
   constexpr int kLocRegs = kCmRegs > 0 ? kCmRegs : 1;
+  // Rows of one vector per lane and every query head in one pass: a wave's
+  // share of up to 64 pages has its row ids in one load and goes through two
+  // register buffers of kStep pages, the next one's rows in flight while one
+  // is scored.  Half of this kernel's time was VALU work and the other half
+  // waits of up to four dependent passes; with the buffers, and two columns
+  // rounded by one instruction (quest_add), 512 segments of up to 512 pages
+  // take 21.2 us per layer instead of 24.7, 8 of 256 pages 12.2 instead of
+  // 16.1.  Steps of 8 pages: 20.9 and 13.5 us.
+  constexpr int kStep = 16;
+  const bool piped = VPL == 1 && a.G <= kG;  // uniform
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ vtx::SelectShared<T> sh;
   __shared__ vtx::BitonicShared<T> bsh;  // cached segments of up to T pages with k <= 32
 
-  const int tid = threadIdx.x;
   const int lane = vtx::lane_id();
   const int wave = vtx::uniform(threadIdx.x / vtx::kWave);
   const int grp = lane / LPR;
@@ -120,7 +124,8 @@ __global__ __launch_bounds__(T, (VPL == 1 ? 4 : (VPL <= 4 ? 2 : 1))) void quest_
   auto first_pass = [&]() {
     share = (n + kWaves - 1) / kWaves;
     share = (share + kRowsPerLoad - 1) / kRowsPerLoad * kRowsPerLoad;
-    if (share > kPass) share = kPass;
+    const int most = piped ? vtx::kWave : kPass;
+    if (share > most) share = most;
     const long long p0 = (long long)wave * share;
     const long long cnt = p0 < n ? min(share, n - p0) : 0;
     my_row = lane < cnt ? a.didx[start + p0 + lane] : -1;
@@ -174,70 +179,127 @@ __global__ __launch_bounds__(T, (VPL == 1 ? 4 : (VPL <= 4 ? 2 : 1))) void quest_
   }
 
   // ---- scores, page maxima and keys of every middle page
-  for (long long p0 = (long long)wave * share; p0 < n; p0 += (long long)kWaves * share) {
-    const int cnt = (int)min(share, n - p0);
-    if (p0 != (long long)wave * share) my_row = lane < cnt ? dseg[p0 + lane] : -1;  // later passes
-    int r = -1;
-    float best = -INFINITY;
-    for (int g0 = 0; g0 < G; g0 += kG) {
-      float xs[kG][VPL][8];
-      // heads past G read head G - 1 and are zeroed by a select (no branch
-      // around the load, which would make the wave wait for it there)
-#pragma unroll
-      for (int gg = 0; gg < kG; ++gg)
-#pragma unroll
-        for (int v = 0; v < VPL; ++v) {
-          const bool in = g0 + gg < G;
-          float f[8];
-          vtx::unpack8(vtx::ld16(qs + (long long)(in ? g0 + gg : G - 1) * D + (v * LPR + col) * 8), f);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) xs[gg][v][e] = in ? f[e] : 0.f;
-        }
-      float sc[kG];
-      vtx::quest_pass_multi<LPR, VPL, kPass, kG>(a.ymax, a.ymin, a.y_rows, D, my_row, cnt, xs, grp, col, &r, sc);
-      if (r >= 0) {
-#pragma unroll
-        for (int gg = 0; gg < kG; ++gg) {
-          if (g0 + gg >= G) break;
-          const uint32_t b = vtx::f32_to_bf16(sc[gg]);
-          a.sum[(start + p0 + r) * G + g0 + gg] = (uint16_t)b;
-          best = fmaxf(best, vtx::bf16_to_f32(b));
-        }
-      }
+  // page maximum `best` at position p of the segment, row id rid
+  auto page_done = [&](long long p, int rid, float best) {
+    const uint32_t ab = vtx::f32_to_bf16(best);
+    const uint32_t key = vtx::score_key(ab);
+    a.aggr[start + p] = (uint16_t)ab;
+    if (cached) {
+      keys[p] = (uint16_t)key;
+      rows[p] = rid;
     }
-    const int my_rid = __shfl(my_row, r < 0 ? 0 : r, vtx::kWave);
+    if (!bitonic) vtx::select_count<T>(key, sh);
+  };
+  // A page whose envelopes this launch rewrites (p and rid uniform): scored
+  // against the envelopes recomputed from the K tile, stored by lane l.
+  auto fresh_page = [&](int l, long long p, int rid) {
     if constexpr (cm_on) {
-      if (n_close > 0) {  // uniform
-        // pages whose envelopes this launch rewrites: scored against the
-        // envelopes recomputed from the K tile, one page at a time per wave,
-        // stored by the lane that stored the first scores
-        uint64_t m = __ballot(vtx::closes_here(cma, closing, r, my_rid));
-        while (m) {  // uniform
-          const int l = __ffsll((long long)m) - 1;
-          m &= m - 1;
-          vtx::U4 emx, emn;
-          vtx::fresh_envelope<LPR>(cma, __builtin_amdgcn_readlane(my_rid, l), grp, col, emx, emn);
-          float fbest = -INFINITY;
-          for (int g = 0; g < G; ++g) {
-            float xg[8];
-            vtx::unpack8(vtx::ld16(qs + (long long)g * D + col * 8), xg);
-            const uint32_t b = vtx::f32_to_bf16(quest_vec<LPR>(emx, emn, xg));
-            if (lane == l) a.sum[(start + p0 + r) * G + g] = (uint16_t)b;
-            fbest = fmaxf(fbest, vtx::bf16_to_f32(b));
+      vtx::U4 emx, emn;
+      vtx::fresh_envelope<LPR>(cma, rid, grp, col, emx, emn);
+      float best = -INFINITY;
+      for (int g = 0; g < G; ++g) {
+        float xg[8];
+        vtx::unpack8(vtx::ld16(qs + (long long)g * D + col * 8), xg);
+        const uint32_t b = vtx::f32_to_bf16(quest_vec<LPR>(emx, emn, xg));
+        if (lane == l) a.sum[(start + p) * G + g] = (uint16_t)b;
+        best = fmaxf(best, vtx::bf16_to_f32(b));
+      }
+      if (lane == l) page_done(p, rid, best);
+    }
+  };
+  // scores of the query heads g0 .. of a page, their maximum into best
+  auto heads_done = [&](long long p, int g0, const float (&sc)[kG], float& best) {
+#pragma unroll
+    for (int gg = 0; gg < kG; ++gg) {
+      if (g0 + gg >= G) break;
+      const uint32_t b = vtx::f32_to_bf16(sc[gg]);
+      a.sum[(start + p) * G + g0 + gg] = (uint16_t)b;
+      best = fmaxf(best, vtx::bf16_to_f32(b));
+    }
+  };
+  // query heads g0 .. g0 + kG (heads past G read head G - 1 and are zeroed by
+  // a select: no branch around the load, which would make the wave wait for
+  // it there)
+  auto load_query = [&](int g0, float (&xs)[kG][VPL][8]) {
+#pragma unroll
+    for (int gg = 0; gg < kG; ++gg)
+#pragma unroll
+      for (int v = 0; v < VPL; ++v) {
+        const bool in = g0 + gg < G;
+        float f[8];
+        vtx::unpack8(vtx::ld16(qs + (long long)(in ? g0 + gg : G - 1) * D + (v * LPR + col) * 8), f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xs[gg][v][e] = in ? f[e] : 0.f;
+      }
+  };
+  if (piped) {  // uniform
+    if constexpr (VPL == 1) {
+      float xv[kG][VPL][8];
+      load_query(0, xv);
+      auto& xs = reinterpret_cast<float(&)[kG][8]>(xv);
+      for (long long p0 = (long long)wave * share; p0 < n; p0 += (long long)kWaves * share) {
+        const int cnt = (int)min(share, n - p0);
+        if (p0 != (long long)wave * share) my_row = lane < cnt ? dseg[p0 + lane] : -1;  // later shares
+        int fill = __builtin_amdgcn_readlane(my_row, 0);
+        if (fill < 0 || fill >= a.y_rows) fill = 0;
+        // the share's pages that are scored afresh, after the others
+        uint64_t fresh = 0;
+        if constexpr (cm_on)
+          if (n_close > 0) fresh = __ballot(vtx::closes_here(cma, closing, lane < cnt ? lane : -1, my_row));
+        vtx::QuestRows<LPR, kStep> ba, bb;
+        auto issue = [&](int at, vtx::QuestRows<LPR, kStep>& b) {
+          vtx::quest_issue<LPR, kStep>(a.ymax, a.ymin, a.y_rows, my_row, fill, at, cnt, grp, col, b);
+        };
+        auto score = [&](int at, const vtx::QuestRows<LPR, kStep>& b) {
+          int r;
+          float sc[kG];
+          vtx::quest_score<LPR, kStep, kG>(b, xs, at, cnt, grp, col, &r, sc);
+          const int rid = __shfl(my_row, (at + r) & (vtx::kWave - 1), vtx::kWave);
+          if (r >= 0 && !(fresh >> (at + r) & 1)) {
+            float best = -INFINITY;
+            heads_done(p0 + at + r, 0, sc, best);
+            page_done(p0 + at + r, rid, best);
           }
-          if (lane == l) best = fbest;
+        };
+        issue(0, ba);
+        for (int at = 0; at < cnt; at += 2 * kStep) {  // uniform
+          issue(at + kStep, bb);
+          score(at, ba);
+          issue(at + 2 * kStep, ba);
+          if (at + kStep < cnt) score(at + kStep, bb);
+        }
+        for (; fresh; fresh &= fresh - 1) {  // uniform
+          const int l = __ffsll((long long)fresh) - 1;
+          fresh_page(l, p0 + l, __builtin_amdgcn_readlane(my_row, l));
         }
       }
     }
-    if (r >= 0) {
-      const uint32_t ab = vtx::f32_to_bf16(best);
-      const uint32_t key = vtx::score_key(ab);
-      a.aggr[start + p0 + r] = (uint16_t)ab;
-      if (cached) {
-        keys[p0 + r] = (uint16_t)key;
-        rows[p0 + r] = my_rid;
+  } else {
+    for (long long p0 = (long long)wave * share; p0 < n; p0 += (long long)kWaves * share) {
+      const int cnt = (int)min(share, n - p0);
+      if (p0 != (long long)wave * share) my_row = lane < cnt ? dseg[p0 + lane] : -1;  // later passes
+      int r = -1;
+      float best = -INFINITY;
+      for (int g0 = 0; g0 < G; g0 += kG) {
+        float xs[kG][VPL][8];
+        load_query(g0, xs);
+        float sc[kG];
+        vtx::quest_pass_multi<LPR, VPL, kPass, kG>(a.ymax, a.ymin, a.y_rows, D, my_row, cnt, xs, grp, col, &r, sc);
+        if (r >= 0) heads_done(p0 + r, g0, sc, best);
       }
-      if (!bitonic) vtx::select_count<T>(key, sh);
+      const int rid = __shfl(my_row, r < 0 ? 0 : r, vtx::kWave);
+      bool done = r < 0;
+      if constexpr (cm_on) {
+        if (n_close > 0) {  // uniform: stored again by the lane that stored the first scores
+          const bool again = vtx::closes_here(cma, closing, r, rid);
+          done |= again;
+          for (uint64_t m = __ballot(again); m; m &= m - 1) {
+            const int l = __ffsll((long long)m) - 1;
+            fresh_page(l, p0 + __builtin_amdgcn_readlane(r, l), __builtin_amdgcn_readlane(rid, l));
+          }
+        }
+      }
+      if (!done) page_done(p0 + r, rid, best);
     }
   }
   __syncthreads();
@@ -470,9 +532,11 @@ int quest_impl(const uint16_t* q, int64_t q_rows, int32_t group_size, const uint
     cma.page_shift = vtx::log2_exact(cms->page_size);
   }
   const vtx::CmArgs* cmp = cm_launch ? &cma : nullptr;
-  if (max_num_pages <= 256) return launch_g<256>(a, cmp, eff_batch_size, lds, s);
-  if (max_num_pages <= 1024) return launch_g<512>(a, cmp, eff_batch_size, lds, s);
-  return launch_g<1024>(a, cmp, eff_batch_size, lds, s);
+  switch (vtx::segment_threads(eff_batch_size, max_num_pages, vtx::device_cu_count())) {
+    case 256: return launch_g<256>(a, cmp, eff_batch_size, lds, s);
+    case 512: return launch_g<512>(a, cmp, eff_batch_size, lds, s);
+    default: return launch_g<1024>(a, cmp, eff_batch_size, lds, s);
+  }
 }
 
 }  // namespace

@@ -43,6 +43,13 @@ __device__ __forceinline__ uint32_t f32_to_bf16(float f) {
 // stays a NaN (its payload is not specified).
 __device__ __forceinline__ float bf16r(float f) { return (float)(__bf16)f; }
 
+// The same for two values by one conversion, packed (lo, hi).
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
+
 // Maps a bf16 bit pattern to a 16-bit unsigned key whose unsigned order is
 // the numeric order of the scores; -0.0 and +0.0 map to the same key.
 __device__ __forceinline__ uint32_t score_key(uint32_t bits16) {

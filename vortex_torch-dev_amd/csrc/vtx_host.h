@@ -31,4 +31,17 @@ inline bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
 
+// Threads per workgroup of the fused indexer kernels with one workgroup per
+// segment (of at most max_pages pages): 4 or 8 waves for up to 256 or 512
+// pages, and past that 16 only where no CU has two workgroups.  Two of 8 waves
+// per CU do one's select while the other's rows arrive; alone on a CU, 16 waves
+// are faster.  Measured per layer, 8 / 16 waves: block-sparse, 512 segments of
+// up to 2048 pages 33.0 / 37.9 us, 256 of up to 1024 pages 16.6 / 14.9; GQA,
+// 320 of up to 1024 pages 23.5 / 28.5, 128 of up to 1024 18.7 / 16.6; Quest,
+// 384 of up to 2048 pages 60.3 / 63.8, 128 of up to 1024 26.4 / 23.8.
+inline int segment_threads(long long segments, long long max_pages, int cus) {
+  if (max_pages <= 256) return 256;
+  return max_pages <= 512 || segments > cus ? 512 : 1024;
+}
+
 }  // namespace vtx

@@ -166,14 +166,29 @@ __device__ __forceinline__ void score_pass_multi(const uint16_t* y, long long y_
                                    [&](const U4 (&rows)[1][VPL], int g) { return dot_row<VPL>(rows[0], xs[g]); });
 }
 
-// Quest page scores (arXiv:2406.10774) of kG fp32 query rows against each
-// position's key envelope (rows of ymax and ymin):
-//   sum_d max(bf16(q_d * max_d), bf16(q_d * min_d))
-// with the lane's partial summed in column order from 0 — the elementwise
-// multiply, maximum and row-sum kernels' arithmetic, in their order.  The
-// maximum is taken before the rounding: rounding is monotonic, so
+// A lane's partial Quest score (arXiv:2406.10774) of one envelope vector (mx,
+// mn: 8 columns each) for its query slice, added to s in column order:
+//   s + sum_e bf16(max(q_e * max_e, q_e * min_e))
+// the elementwise multiply, maximum and row-sum kernels' arithmetic, in their
+// order.  The maximum is taken before the rounding: rounding is monotonic, so
 // bf16(max(a, b)) = max(bf16(a), bf16(b)) for all a, b (a NaN product is
-// dropped by the maximum either way), with one conversion instead of two.
+// dropped by the maximum either way), with one conversion instead of two, and
+// one instruction converts two columns.
+__device__ __forceinline__ float quest_add(const U4& mx, const U4& mn, const float (&xs)[8], float s) {
+  const uint32_t a[4] = {mx.x, mx.y, mx.z, mx.w}, b[4] = {mn.x, mn.y, mn.z, mn.w};
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float lo = fmaxf(xs[2 * w] * bf16_lo(a[w]), xs[2 * w] * bf16_lo(b[w]));
+    const float hi = fmaxf(xs[2 * w + 1] * bf16_hi(a[w]), xs[2 * w + 1] * bf16_hi(b[w]));
+    const uint32_t pair = bf16_pair(lo, hi);
+    s += bf16_lo(pair);
+    s += bf16_hi(pair);
+  }
+  return s;
+}
+
+// Quest page scores of kG fp32 query rows against each position's key
+// envelope (rows of ymax and ymin).
 template <int LPR, int VPL, int kPass, int kG>
 __device__ __forceinline__ void quest_pass_multi(const uint16_t* ymax, const uint16_t* ymin, long long y_rows, int D,
                                                  int my_row, int cnt, const float (&xs)[kG][VPL][8], int grp,
@@ -183,16 +198,71 @@ __device__ __forceinline__ void quest_pass_multi(const uint16_t* ymax, const uin
                                    [&](const U4 (&rows)[2][VPL], int g) {
                                      float s = 0.f;
 #pragma unroll
-                                     for (int v = 0; v < VPL; ++v) {
-                                       float mx[8], mn[8];
-                                       unpack8(rows[0][v], mx);
-                                       unpack8(rows[1][v], mn);
-#pragma unroll
-                                       for (int e = 0; e < 8; ++e)
-                                         s += bf16r(fmaxf(xs[g][v][e] * mx[e], xs[g][v][e] * mn[e]));
-                                     }
+                                     for (int v = 0; v < VPL; ++v) s = quest_add(rows[0][v], rows[1][v], xs[g][v], s);
                                      return s;
                                    });
+}
+
+// quest_pass_multi in two halves for rows of one vector per lane, so that the
+// next pass's rows can be in flight while one is scored: quest_issue loads
+// positions first .. first + kPass of a wave's positions (lane l of my_row: the
+// row id of its l-th position; at and past cnt a lane reads row `fill` again,
+// which no result uses: every load is issued, so a wait for one pass's rows
+// waits for no other's), quest_score gives row_pass's results from them.
+template <int LPR, int kPass>
+struct QuestRows {
+  static constexpr int kSlots = kPass / (kWave / LPR);
+  U4 mx[kSlots], mn[kSlots];
+  bool live[kSlots];
+};
+
+template <int LPR, int kPass>
+__device__ __forceinline__ void quest_issue(const uint16_t* ymax, const uint16_t* ymin, long long y_rows, int my_row,
+                                            int fill, int first, int cnt, int grp, int col, QuestRows<LPR, kPass>& b) {
+#pragma unroll
+  for (int i = 0; i < QuestRows<LPR, kPass>::kSlots; ++i) {
+    const int at = first + i * (kWave / LPR) + grp;
+    const int row = __shfl(my_row, at & (kWave - 1), kWave);
+    b.live[i] = at < cnt && row >= 0 && row < y_rows;
+    const long long off = (long long)(b.live[i] ? row : fill) * (LPR * 8) + col * 8;
+    b.mx[i] = ld16_stream(ymax + off);
+    b.mn[i] = ld16_stream(ymin + off);
+  }
+}
+
+template <int LPR, int kPass, int kG>
+__device__ __forceinline__ void quest_score(const QuestRows<LPR, kPass>& b, const float (&xs)[kG][8], int first,
+                                            int cnt, int grp, int col, int* r, float (&sc)[kG]) {
+  constexpr int kSlots = QuestRows<LPR, kPass>::kSlots;
+  float acc[kG][kSlots];
+#pragma unroll
+  for (int i = 0; i < kSlots; ++i)
+#pragma unroll
+    for (int g = 0; g < kG; ++g) {
+      const float s = quest_add(b.mx[i], b.mn[i], xs[g], 0.f);
+      acc[g][i] = b.live[i] ? s : 0.f;
+    }
+  // (row_pass's reduce-scatter; shared as a function, it cost row_pass registers)
+#pragma unroll
+  for (int g = 0; g < kG; ++g) {
+#pragma unroll
+    for (int half = kSlots / 2, stride = LPR / 2; half >= 1; half >>= 1, stride >>= 1) {
+      const bool upper = (col & stride) != 0;
+#pragma unroll
+      for (int t = 0; t < half; ++t) {
+        const float send = upper ? acc[g][t] : acc[g][t + half];
+        const float keep = upper ? acc[g][t + half] : acc[g][t];
+        acc[g][t] = keep + xshfl(send, stride);
+      }
+    }
+    constexpr int kShare = LPR / kSlots;  // lanes holding the same slot
+#pragma unroll
+    for (int d = kShare / 2; d >= 1; d >>= 1) acc[g][0] += xshfl(acc[g][0], d);
+    sc[g] = acc[g][0];
+  }
+  constexpr int kShare = LPR / kSlots;
+  const int pos = (col / kShare) * (kWave / LPR) + grp;
+  *r = ((col % kShare) == 0 && first + pos < cnt) ? pos : -1;
 }
 
 // score_pass with the query slice as packed bf16 pairs (dot_row_packed:
