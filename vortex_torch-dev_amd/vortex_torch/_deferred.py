@@ -334,31 +334,39 @@ def take_carry_envelope(ya: torch.Tensor, yb: torch.Tensor):
     return p, p.output_of(_hip.REDUCE_MAX), p.output_of(_hip.REDUCE_MIN)
 
 
-@contextlib.contextmanager
-def scope(active: bool, kind: str = "indexer"):
-    """Deferral scope; flushes everything still pending on exit.  kind
-    "cache" (forward_cache) may leave a page-finish mean as the carry;
-    kind "indexer" (forward_indexer) may consume it and launches it at exit
-    if it did not."""
-    if active and kind == "cache":
-        flush_carry()
-    prev = current_scope()
-    sc = Scope() if active else None
-    _tls.scope = sc
-    try:
-        yield sc
-    finally:
-        _tls.scope = prev
-        if sc is not None:
-            if (kind == "cache" and _carry_enabled() and len(sc.pending) == 1
-                    and getattr(sc.pending[0], "carryable", lambda: False)()):
-                p = sc.pending.pop()
+class scope:
+    """Deferral scope (a context manager); flushes everything still pending on
+    exit.  kind "cache" (forward_cache) may leave a page-finish mean as the
+    carry; kind "indexer" (forward_indexer) may consume it and launches it at
+    exit if it did not."""
+
+    __slots__ = ("active", "kind", "prev", "sc")
+
+    def __init__(self, active: bool, kind: str = "indexer"):
+        self.active, self.kind = active, kind
+
+    def __enter__(self) -> Optional[Scope]:
+        if self.active and self.kind == "cache":
+            flush_carry()
+        self.prev = current_scope()
+        self.sc = _tls.scope = Scope() if self.active else None
+        return self.sc
+
+    def __exit__(self, *exc) -> None:
+        sc = self.sc
+        _tls.scope = self.prev
+        if sc is None:
+            return
+        if self.kind == "cache" and len(sc.pending) == 1:
+            p = sc.pending[0]
+            if getattr(p, "carryable", lambda: False)() and _carry_enabled():
+                sc.pending.pop()
                 st = _stream_of(p.x.device)
                 _install_capture_hooks()  # (only while something is carried)
                 _tls.carry = (p, st, _capture_of(st))
-            sc.flush()
-            if kind == "indexer":
-                flush_carry()
+        sc.flush()
+        if self.kind == "indexer":
+            flush_carry()
 
 
 def flush_all() -> None:
@@ -475,14 +483,16 @@ def materialize(t):
     return t
 
 
-def plain(t: torch.Tensor) -> torch.Tensor:
-    """`t` as a plain torch.Tensor over the same storage, without running its
-    subclass hooks (a recorded launch must not flush the scope it runs in).
-    The result does not keep `t`'s Python object alive (``as_subclass`` would:
-    its view refers back to `t`), so a recorded launch holding it does not
-    make an elided result look observed."""
+def plain(*ts: torch.Tensor):
+    """Each tensor as a plain torch.Tensor over the same storage (a list; of one
+    tensor, the tensor), without running its subclass hooks (a recorded launch
+    must not flush the scope it runs in).  The results do not keep the
+    originals' Python objects alive (``as_subclass`` would: its view refers back
+    to them), so a recorded launch holding one does not make an elided result
+    look observed."""
     with torch._C.DisableTorchFunctionSubclass():
-        return torch.Tensor._make_subclass(torch.Tensor, t, require_grad=False)
+        out = [torch.Tensor._make_subclass(torch.Tensor, t, require_grad=False) for t in ts]
+    return out if len(out) > 1 else out[0]
 
 
 def _install_launch_hook() -> None:

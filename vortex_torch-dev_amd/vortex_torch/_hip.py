@@ -177,7 +177,9 @@ def load_library(path: os.PathLike | str | None = None) -> ctypes.CDLL:
 def _plain(t):
     """The same tensor without its subclass: layout-tagged and deferred tensors
     are passed to the kernels by pointer, without running their torch hooks."""
-    if isinstance(t, torch.Tensor) and type(t) is not torch.Tensor:
+    if type(t) is torch.Tensor:
+        return t
+    if isinstance(t, torch.Tensor):
         with torch._C.DisableTorchFunctionSubclass():
             return t.as_subclass(torch.Tensor)
     if isinstance(t, (list, tuple)):
@@ -214,16 +216,16 @@ def set_pre_launch_hook(fn) -> None:
 def _require_gpu(*tensors: torch.Tensor) -> torch.device:
     if _pre_launch is not None:
         _pre_launch()
-    dev = None
+    dev, index = None, -1
     for t in tensors:
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 f"vortex_torch: HIP kernels need GPU tensors, got a tensor on {t.device} "
                 "(there is no CPU implementation)"
             )
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, t.get_device()
+        elif t.get_device() != index:
             raise RuntimeError(f"vortex_torch: tensors on different devices ({dev} vs {t.device})")
     return dev
 
@@ -236,8 +238,17 @@ def _req(t: torch.Tensor, dtype: torch.dtype, name: str) -> torch.Tensor:
     return t
 
 
+# The current stream's handle without a torch.cuda.Stream object around it, and
+# the current device without the initialisation check (the callers hold GPU
+# tensors): together they were a quarter of an eager call's host time.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    if _raw_stream is None or dev.index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(dev.index)
 
 
 def stream_capture_id(stream) -> int:
@@ -268,7 +279,7 @@ class _on_device:
         self.prev = None
 
     def __enter__(self):
-        cur = torch.cuda.current_device()
+        cur = _current_device()
         idx = self.dev.index if self.dev.index is not None else cur
         if idx != cur:
             self.prev = cur
@@ -985,9 +996,10 @@ def set_kv_buffer(k_cache, v_cache, new_k, new_v, loc, page_size: int) -> None:
     _req(loc, torch.int64, "loc")
     if new_k.dim() != 3 or new_v.shape != new_k.shape:
         raise RuntimeError("vortex_torch: new_k and new_v must both be [nnz, num_kv_heads, head_dim]")
+    dtype = new_k.dtype
     for t, n in ((k_cache, "k_cache"), (v_cache, "v_cache"), (new_k, "new_k"), (new_v, "new_v")):
-        if t.dtype != new_k.dtype:
-            raise RuntimeError(f"vortex_torch: {n} is {t.dtype}, the new tokens are {new_k.dtype}")
+        if t.dtype != dtype:
+            raise RuntimeError(f"vortex_torch: {n} is {t.dtype}, the new tokens are {dtype}")
         if not t.is_contiguous():
             raise RuntimeError(f"vortex_torch: {n} must be contiguous")
     nnz, H, D = (int(s) for s in new_k.shape)

@@ -95,7 +95,7 @@ class _PendingPageReduce(_deferred.Pending):
         (vtx_indexer_fused_cmean and its GQA / Quest forms): a decode-sized
         CMean, or CMax + CMin, (dim 1) of [page_size, D] tiles into bf16
         [rows, 1, D] pools."""
-        if self.done or self.dim != 1 or self.carry_kind() is None:
+        if self.done or self.dim != 1 or self.loc.numel() > self.CARRY_MAX_LOC or self.carry_kind() is None:
             return False
         x = self.x
         for out in self.outs:
@@ -106,7 +106,7 @@ class _PendingPageReduce(_deferred.Pending):
                         and int(x.shape[2]) == int(out.shape[2])):
                     return False
         with torch._C.DisableTorchFunctionSubclass():
-            return int(x.shape[1]) == int(self.ctx.page_size) and self.loc.numel() <= self.CARRY_MAX_LOC
+            return int(x.shape[1]) == int(self.ctx.page_size)
 
     def _run(self) -> None:
         c = self.ctx
@@ -126,7 +126,7 @@ def _record_page_reduce(x, output, loc, ctx: Context, dim: int, reduce_type: Red
         return False
     if not _recordable_operands(x, output, loc):
         return False
-    xp, op, lp = _deferred.plain(x), _deferred.plain(output), _deferred.plain(loc)
+    xp, op, lp = _deferred.plain(x, output, loc)
     last = sc.pending[-1] if sc.pending else None
     if not (isinstance(last, _PendingPageReduce) and last.accepts(xp, op, lp, ctx, dim)):
         last = _PendingPageReduce(xp, lp, ctx, dim)
@@ -202,10 +202,10 @@ class Reduce(vOp):
 
     def execute(self, x: torch.Tensor, output: Optional[torch.Tensor], loc: torch.Tensor,
                 ctx: Context) -> torch.Tensor:
-        p = self._prefix()
-        assert self.impl is not None, f"{p}called before profile() (impl is None)"
+        assert self.impl is not None, f"{self._prefix()}called before profile() (impl is None)"
         if output is None:
-            assert self.output_buffer is not None, f"{p}internal output buffer is None; did profile() run?"
+            assert self.output_buffer is not None, (
+                f"{self._prefix()}internal output buffer is None; did profile() run?")
             output = self.output_buffer
         if self.impl is reduce_pp and _record_page_reduce(x, output, loc, ctx, self.dim, self.reduce_type):
             return output
