@@ -385,3 +385,27 @@ def test_reduce_c4_burst_full_size(gpu):
             np.testing.assert_array_equal(got, exp)
         else:
             np.testing.assert_allclose(O.bf16_to_f32(got), O.bf16_to_f32(exp), rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("nnz", [767, 768, 769, 1024, 5003])
+@pytest.mark.parametrize("heads,page,cols", [(8, 16, 128), (1, 16, 64), (3, 4, 128), (8, 1, 256), (2, 32, 128),
+                                             (5, 16, 576)])
+def test_reduce_burst_equals_small_calls(gpu, nnz, heads, page, cols):
+    """A burst's tiles, shared by as many workgroups as its blocks of loc
+    entries close pages for, get the bits of calls over 256 entries each (one
+    block, one tile per wave), at the entry count where a burst begins and at
+    ragged ends, for every way a block's tiles are dealt."""
+    pool = 260 + nnz // page
+    g = torch.Generator().manual_seed(nnz + heads)
+    loc = torch.randperm(pool * page, generator=g)[:nnz]
+    loc[::2] = loc[::2] // page * page + page - 1  # half of the entries close a page
+    loc = loc.to(gpu)
+    k = W.randn_bf16((pool * heads, page, cols), 5, gpu)
+    types = [_hip.REDUCE_MEAN, _hip.REDUCE_MAX]
+    whole, parts = ([torch.full((pool * heads, 1, cols), -3.0, dtype=torch.bfloat16, device=gpu) for _ in types]
+                    for _ in range(2))
+    _hip.page_reduce_multi(k, whole, types, loc, heads, page)
+    for at in range(0, nnz, 256):
+        _hip.page_reduce_multi(k, parts, types, loc[at:at + 256].contiguous(), heads, page)
+    for a, b in zip(whole, parts):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))

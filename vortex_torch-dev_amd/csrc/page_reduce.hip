@@ -50,6 +50,9 @@ __device__ __forceinline__ void store_one(const ReduceArgs& a, int o, long long 
     reinterpret_cast<uint32_t*>(a.out[o])[elem] = bits << 16;
 }
 
+constexpr int kLaneRows = 16;    // rows of the tallest tile that one lane per column vector reduces
+constexpr int kBurstBlocks = 4;  // from so many blocks of loc entries on, a burst (1024 entries and more)
+
 // The pages closed by this block's 256 loc entries (the workgroups that share
 // a block of entries split its tiles by index, so they all see the same list).
 __device__ __forceinline__ int collect_pages(const ReduceArgs& a, long long* first_row, int* wave_count) {
@@ -79,7 +82,7 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_vec_kernel(ReduceArgs a)
   if constexpr (vtx::lane_tiles_fit<LPR, NEED>()) {
     // (a decode-sized loc, whose few tiles are spread over several
     // workgroups, keeps one tile per wave: more waves share the latency)
-    if (R <= 16 && gridDim.y == 1) {  // uniform
+    if (R <= kLaneRows && gridDim.x >= kBurstBlocks) {  // uniform
       constexpr int kSlots = vtx::kWave / LPR;  // tiles per wave at once; lane group grp takes slot grp
       for (int t0 = (blockIdx.y * kWavesPerBlock + wave) * kSlots; t0 < tiles;
            t0 += gridDim.y * kWavesPerBlock * kSlots) {
@@ -250,17 +253,30 @@ int launch_reduce(ReduceArgs& a, int dim, void* stream) {
   const long long blocks = (a.nnz + kThreads - 1) / kThreads;
   if (blocks > 0x7fffffffLL) return vtx::fail(VTX_E_INVALID, "page_reduce: loc too long");
   hipStream_t s = vtx::as_stream(stream);
-  // Few loc entries (a decode step): the closed pages' tiles of one block of
-  // entries are spread over up to 16 workgroups (each rescans the same
-  // entries), so the tiles are reduced side by side rather than by 4 waves.
-  long long split = (512 + blocks - 1) / blocks;
-  if (split > 16) split = 16;
-  if (split < 1) split = 1;
-  const dim3 grid((unsigned)blocks, (unsigned)split);
   const bool vec = dim == 1 && (a.cols % 8 == 0) && vtx::aligned16(a.x) && out_aligned;
   const int lpr = a.cols / 8;
   int need = 0;
   for (int o = 0; o < a.n_out; ++o) need |= need_of(a.out_type[o]);
+  // The closed pages' tiles of one block of entries are shared by `split`
+  // workgroups (each rescans the same entries).  Few loc entries (a decode
+  // step): up to 16, so the tiles are reduced side by side rather than by 4
+  // waves.  A burst: enough that one round of a workgroup's waves takes its
+  // share of the tiles that a block of whole pages closes, so that scans and
+  // first loads of some overlap the tiles of others and the last workgroups to
+  // run are short.  65,536 pages of 8 heads, CMean + CMax: 514 us with one
+  // workgroup per block, 501 with two, 495 with four; 4,096 pages: 78 -> 34
+  // us (before, sharing also meant one tile per wave); one head (16 tiles per
+  // block), 32,768 pages: 20.7 us with one, 28 with eight.
+  long long split;
+  if (blocks < kBurstBlocks) {
+    split = 16;
+  } else {
+    const bool lane = vec && a.rows_per_tile <= kLaneRows && (lpr == 8 || lpr == 16 || lpr == 32 || lpr == 64);
+    const long long per_round = (long long)kWavesPerBlock * (lane ? vtx::kWave / lpr : 1);
+    split = (long long)kThreads / a.page * a.heads / per_round;
+    split = split < 1 ? 1 : (split > 16 ? 16 : split);
+  }
+  const dim3 grid((unsigned)blocks, (unsigned)split);
   if (vec && lpr == 8) {
     launch_vec<8>(a, need, grid, s);
   } else if (vec && lpr == 16) {
