@@ -821,3 +821,41 @@ def test_decode_attention_split_segments(gpu, name):
                                         D, P, 1.0 / np.sqrt(D), torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     np.testing.assert_allclose(_f(_bits(got)), _f(_bits(whole)), rtol=2 ** -7, atol=1e-4)
+
+
+# (request lengths, kv heads, page size): batch edges; a segment of more than 64
+# batches per wave, whole; one of more than 2048 pages, whole; pages of 48
+_MATRIX_TABLES = {
+    "edges": ([1, 15, 16, 17, 31, 33, 64, 65, 0, 257], 2, 16),
+    "long": ([9000] + [1 + i % 20 for i in range(39)], 1, 16),
+    "unstaged": ([33000] + [1 + i % 20 for i in range(119)], 1, 16),
+    "page48": ([700, 47, 49, 1000], 2, 48),
+}
+
+
+@pytest.mark.parametrize("name", sorted(_MATRIX_TABLES))
+@pytest.mark.parametrize("G,D", [(3, 64), (4, 128), (8, 128), (5, 64)])
+def test_decode_attention_many_heads(gpu, name, G, D):
+    """Three and more query heads per kv head (the matrix cores' kernel):
+    within the bf16 rounding of the result of the oracle, whatever the slots
+    of the last page past the segment hold."""
+    from vortex_torch.decode_attention import paged_decode_attention
+    from vortex_torch.indexer.utils_sglang import plan_decode
+
+    lens, H, P = _MATRIX_TABLES[name]
+    pool = sum((n + P - 1) // P for n in lens) + 3
+    batch = W.make_batch(lens, pool_pages=pool, seed=43, page_size=P, num_kv_heads=H, group_size=G, head_dim=D)
+    ic, _ = W.make_contexts(batch, gpu)
+    b = batch.to(gpu)
+    plan_decode(b.seq_lens, b.req_to_token, b.req_indices, ic)
+    q, k, v = _attn_inputs(batch, gpu, G, D, 17)
+    args = (ic.dense_kv_indptr, ic.dense_kv_indices, ic.kv_last_page_len)
+    exp = O.paged_decode_attention(_bits(q), _bits(k), _bits(v), *[_np(t) for t in args], len(lens), H,
+                                   1.0 / np.sqrt(D))
+    for pages, n in zip(batch.pages, lens):
+        if n % P:
+            rows = int(pages[-1]) * H
+            k[rows:rows + H, n % P:] = float("nan")
+            v[rows:rows + H, n % P:] = float("inf")
+    o = paged_decode_attention(q, k, v, *args, len(lens), H)
+    np.testing.assert_allclose(_f(_bits(o)), _f(exp), rtol=2 ** -7, atol=1e-4)

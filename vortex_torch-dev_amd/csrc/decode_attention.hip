@@ -12,7 +12,9 @@
 //
 // One workgroup per segment, or per chunk of a segment where segments are few
 // and long (the chunks' partial outputs then combined by a second launch);
-// 8 waves, or 4 for wide G x D.  The segment's
+// 8 waves, or 4 for wide G x D.  Three and more query heads take the matrix
+// cores (decode_attention_mfma_kernel); what follows describes the VALU kernel
+// and holds for both where it speaks of batches and buffers.  The segment's
 // page rows are staged in LDS first (one load per page, up to kPageCap
 // pages; longer segments read them from the table), so each batch of a
 // wave costs one memory round trip: a wave takes every kWaves-th batch of
@@ -21,9 +23,7 @@
 // next batch's K and V loads
 // before it computes on the current one (two register buffers).  It keeps a
 // running max and per-lane partial sums (online softmax); the waves'
-// (max, sum, accumulator) are merged in LDS.  At decode batch sizes the
-// q . K products are G rows against a few hundred tokens: HBM-bound, so the
-// kernel runs on the VALU.
+// (max, sum, accumulator) are merged in LDS.
 #include "vtx_device.h"
 #include "vtx_host.h"
 
@@ -115,6 +115,80 @@ __device__ __forceinline__ uint32_t longest_segment(const AttnArgs& a, uint32_t*
   return mx;
 }
 
+// What a workgroup attends to: a segment, or one chunk of a split one.
+struct Span {
+  int seg, chunk, chunks;
+  long long start, pages;  // its pages in the table
+  int tokens;              // 0: an empty segment
+};
+
+// The workgroup's span; false for a chunk past the segment's last.  Every
+// thread of the workgroup calls it and gets the same answer.
+template <bool kSplit, int T>
+__device__ __forceinline__ bool attn_span(const AttnArgs& a, uint32_t* red, Span& sp) {
+  const int P = a.P;
+  sp.seg = kSplit ? (int)(blockIdx.x % (uint32_t)a.segments) : (int)blockIdx.x;
+  sp.chunk = kSplit ? (int)(blockIdx.x / (uint32_t)a.segments) : 0;
+  sp.chunks = 1;
+  sp.start = a.indptr[sp.seg];
+  sp.pages = (long long)a.indptr[sp.seg + 1] - sp.start;
+  sp.tokens = 0;
+  if (sp.pages > 0 && sp.start >= 0 && sp.start + sp.pages <= a.indices_len && a.rows > 0) {
+    int last = a.last_len[sp.seg];
+    last = last < 0 ? 0 : (last > P ? P : last);
+    const long long t = (sp.pages - 1) * P + last;
+    sp.tokens = t < (1LL << 30) ? (int)t : 0;  // (token indices, with the prefetch past the end, fit an int)
+    if constexpr (kSplit) {
+      if (sp.tokens > 0) {
+        const Chunks c =
+            chunks_of(a, (uint32_t)sp.pages, longest_segment<T>(a, red), a.indptr[0], a.indptr[a.segments]);
+        sp.chunks = (int)c.count;
+        if (sp.chunk < sp.chunks) {  // this chunk's pages as a segment of their own
+          const int p0 = sp.chunk * (int)c.pages;
+          const int p1 = min((int)sp.pages, p0 + (int)c.pages);
+          sp.tokens = (p1 == (int)sp.pages ? sp.tokens : p1 * P) - p0 * P;
+          sp.start += p0;
+          sp.pages = p1 - p0;
+        }
+      }
+    }
+  }
+  return sp.chunk < sp.chunks;
+}
+
+// The waves' (max, sum, output) merged, one thread per (g, column): the
+// result, or for a split segment the chunk's share for the combine kernel.
+template <int kWaves, int kG, int kD, bool kSplit, int T>
+__device__ __forceinline__ void attn_merge(const AttnArgs& a, const Span& sp, const float (*s_m)[kG],
+                                           const float (*s_l)[kG], const float (*s_acc)[kG][kD]) {
+  const int G = a.G;
+  for (int idx = threadIdx.x; idx < G * kD; idx += T) {
+    const int g = idx / kD;
+    const int d = idx - g * kD;
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, s_m[w][g]);
+    float L = 0.f, O = 0.f;
+    if (M != -INFINITY) {
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const float f = __expf(s_m[w][g] - M);
+        L = fmaf(s_l[w][g], f, L);
+        O = fmaf(s_acc[w][g][d], f, O);
+      }
+    }
+    if constexpr (kSplit) {
+      if (sp.chunks > 1) {  // uniform
+        const long long row = ((long long)sp.seg * a.nsplit + sp.chunk) * G + g;
+        a.acc[row * kD + d] = O;
+        if (d == 0) a.ml[row] = float2{M, L};
+        continue;
+      }
+    }
+    a.o[((long long)sp.seg * G + g) * kD + d] = (uint16_t)vtx::f32_to_bf16(L > 0.f ? O / L : 0.f);
+  }
+}
+
 // Threads per workgroup: 8 waves where a wave's registers fit 128 (rows of
 // one 16-byte vector per lane, at most two query heads), else 4.
 template <int LPR, int VPL, int kG>
@@ -141,8 +215,6 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
   __shared__ float s_l[kWaves][kG];
   __shared__ float s_acc[kWaves][kG][LPR * VPL * 8];
 
-  const int seg = kSplit ? (int)(blockIdx.x % (uint32_t)a.segments) : (int)blockIdx.x;
-  const int chunk = kSplit ? (int)(blockIdx.x / (uint32_t)a.segments) : 0;
   const int tid = threadIdx.x;
   const int wave = vtx::uniform(tid / vtx::kWave);
   const int lane = vtx::lane_id();
@@ -150,32 +222,10 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
   const int col = lane % LPR;
   const int G = a.G, D = a.D, P = a.P;
 
-  long long start = a.indptr[seg];
-  long long m = (long long)a.indptr[seg + 1] - start;
-  int T_tok = 0;  // tokens of the segment (of the chunk)
-  int nchunks = 1;
-  if (m > 0 && start >= 0 && start + m <= a.indices_len && a.rows > 0) {
-    int last = a.last_len[seg];
-    last = last < 0 ? 0 : (last > P ? P : last);
-    const long long t = (m - 1) * P + last;
-    T_tok = t < (1LL << 30) ? (int)t : 0;  // (token indices, with the prefetch past the end, fit an int)
-    if constexpr (kSplit) {
-      if (T_tok > 0) {
-        const Chunks c = chunks_of(a, (uint32_t)m, longest_segment<T>(a, s_red), a.indptr[0], a.indptr[a.segments]);
-        nchunks = (int)c.count;
-        if (chunk < nchunks) {  // this chunk's pages as a segment of their own
-          const int p0 = chunk * (int)c.pages;
-          const int p1 = min((int)m, p0 + (int)c.pages);
-          T_tok = (p1 == (int)m ? T_tok : p1 * P) - p0 * P;
-          start += p0;
-          m = p1 - p0;
-        }
-      }
-    }
-  }
-  if constexpr (kSplit) {
-    if (chunk >= nchunks) return;  // uniform
-  }
+  Span sp;
+  if (!attn_span<kSplit, T>(a, s_red, sp)) return;  // uniform
+  const int seg = sp.seg, T_tok = sp.tokens;
+  const long long start = sp.start, m = sp.pages;
   // query slice of this lane (columns (v * LPR + col) * 8 .. + 8), requested
   // first so that it arrives with the page rows; heads past G read head
   // G - 1 and are zeroed by a select (no branch around the load, which would
@@ -333,32 +383,256 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
     }
   }
   __syncthreads();
-  // one thread per (g, column) writes the merged output
-  for (int idx = tid; idx < G * D; idx += T) {
-    const int g = idx / D;
-    const int d = idx - g * D;
-    float M = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, s_m[w][g]);
-    float L = 0.f, O = 0.f;
-    if (M != -INFINITY) {
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float f = __expf(s_m[w][g] - M);
-        L = fmaf(s_l[w][g], f, L);
-        O = fmaf(s_acc[w][g][d], f, O);
-      }
-    }
-    if constexpr (kSplit) {
-      if (nchunks > 1) {  // uniform: for the combine kernel
-        const long long row = ((long long)seg * a.nsplit + chunk) * G + g;
-        a.acc[row * D + d] = O;
-        if (d == 0) a.ml[row] = float2{M, L};
-        continue;
-      }
-    }
-    a.o[((long long)seg * G + g) * D + d] = (uint16_t)vtx::f32_to_bf16(L > 0.f ? O / L : 0.f);
+  attn_merge<kWaves, kG, LPR * VPL * 8, kSplit, T>(a, sp, s_m, s_l, s_acc);
+}
+
+// More than two query heads, rows of 64 or 128 columns, pages of a multiple of
+// 16 tokens: the scores on the matrix cores.
+//
+// With many heads the VALU sets the kernel above's time: dot products with a
+// lane tree each and an exponential per token and head in every lane.  Here a
+// wave takes 16 consecutive tokens per batch, S^T = K Q^T as kD / 32 steps of
+// v_mfma_f32_16x16x32_bf16 (bf16 products, fp32 sums): A holds the tokens' rows
+// (lane l: token l % 16, 16 bytes of its row per step), B the query heads
+// (lane l: head l % 16, zero past G), and lane l ends with tokens
+// 4 (l / 16) + r, r < 4, of head l % 16.  One exponential per lane then serves
+// 16 heads.  The probabilities stay in fp32: for P V, lane l takes columns
+// (l % 16) * kE .. of V's rows of the same four tokens and reads head g's
+// probability from lane g of its 16-lane row (a DPP row broadcast), so P V is
+// kE fused multiply-adds per token and head, with no transposition and no
+// rounding.  A batch lies in one page, so its row is uniform.
+//
+// Per layer, D 128, VALU / matrix: 8 heads, 128 segments of 1k to 16k tokens
+// 280 / 135 us, 512 of 2048 182 / 90; 4 heads 155 / 121 and 110 / 86, 64 segments
+// of 512 tokens 23.5 / 14.2.  Error against 64 bits the same (the result's own
+// rounding).  With two heads the VALU keeps up with the card and its wider
+// loads (a token's 256 bytes by 16 lanes, here 64 by 4) win: 128 segments of 1k
+// to 16k 112 us, 125 here; so 1 and 2 heads stay there.  8 waves instead of 4
+// were slower (8 heads' registers leave one such workgroup per CU).
+constexpr int kMfmaThreads = 256;
+// Waves per SIMD that the registers are limited to.
+template <int kG>
+constexpr int mfma_waves() {
+  return kG <= 4 ? 3 : 2;
+}
+
+template <int kG>
+__device__ __forceinline__ float row_broadcast(float v, int g) {
+  static_assert(kG <= 8, "heads of a row broadcast");
+  const int x = (int)__float_as_uint(v);
+  int y = 0;
+  switch (g) {  // (compile-time constants after unrolling)
+    case 0: y = __builtin_amdgcn_update_dpp(0, x, 0x150, 0xf, 0xf, false); break;
+    case 1: y = __builtin_amdgcn_update_dpp(0, x, 0x151, 0xf, 0xf, false); break;
+    case 2: y = __builtin_amdgcn_update_dpp(0, x, 0x152, 0xf, 0xf, false); break;
+    case 3: y = __builtin_amdgcn_update_dpp(0, x, 0x153, 0xf, 0xf, false); break;
+    case 4: y = __builtin_amdgcn_update_dpp(0, x, 0x154, 0xf, 0xf, false); break;
+    case 5: y = __builtin_amdgcn_update_dpp(0, x, 0x155, 0xf, 0xf, false); break;
+    case 6: y = __builtin_amdgcn_update_dpp(0, x, 0x156, 0xf, 0xf, false); break;
+    default: y = __builtin_amdgcn_update_dpp(0, x, 0x157, 0xf, 0xf, false); break;
   }
+  return __uint_as_float((uint32_t)y);
+}
+
+// kE consecutive bf16 values of a V row: 16 bytes (kE 8) or 8 (kE 4).
+template <int kE>
+struct VRow {
+  uint32_t w[kE / 2];
+};
+template <int kE>
+__device__ __forceinline__ VRow<kE> load_v(const uint16_t* p) {
+  VRow<kE> r;
+  if constexpr (kE == 8) {
+    const vtx::U4 t = vtx::ld16_stream(p);
+    r.w[0] = t.x;
+    r.w[1] = t.y;
+    r.w[2] = t.z;
+    r.w[3] = t.w;
+  } else {
+    typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+    const v2u t = __builtin_nontemporal_load(reinterpret_cast<const v2u*>(p));
+    r.w[0] = t.x;
+    r.w[1] = t.y;
+  }
+  return r;
+}
+
+template <int kD, int kG, bool kSplit>
+__global__ __launch_bounds__(kMfmaThreads, mfma_waves<kG>()) void decode_attention_mfma_kernel(AttnArgs a) {
+  typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int T = kMfmaThreads;
+  constexpr int kWaves = T / vtx::kWave;
+  constexpr int kSteps = kD / 32;  // matrix steps per score
+  constexpr int kE = kD / 16;      // V columns per lane
+  constexpr int kTok = 16;         // tokens per batch
+  __shared__ int32_t s_rows[kPageCap];
+  __shared__ uint32_t s_red[kWaves];
+  __shared__ float s_m[kWaves][kG];
+  __shared__ float s_l[kWaves][kG];
+  __shared__ float s_acc[kWaves][kG][kD];
+
+  const int tid = threadIdx.x;
+  const int wave = vtx::uniform(tid / vtx::kWave);
+  const int lane = vtx::lane_id();
+  const int quad = lane / 16;
+  const int l16 = lane % 16;
+  const int G = a.G, P = a.P;
+
+  Span sp;
+  if (!attn_span<kSplit, T>(a, s_red, sp)) return;  // uniform
+  const int T_tok = sp.tokens;
+
+  // the query heads as the B operand, requested first
+  vtx::U4 qf[kSteps];
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s)
+    qf[s] = vtx::ld16(a.q + ((long long)sp.seg * G + (l16 < G ? l16 : G - 1)) * kD + s * 32 + quad * 8);
+
+  // the segment's page rows (-1: outside the pool)
+  const bool staged = sp.pages <= kPageCap;
+  if (staged && T_tok > 0) {
+    for (int i = tid; i < (int)sp.pages; i += T) {
+      const int r = a.indices[sp.start + i];
+      s_rows[i] = (r >= 0 && r < a.rows) ? r : -1;
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s)
+    if (l16 >= G) qf[s] = vtx::U4{0u, 0u, 0u, 0u};
+
+  float mx = -INFINITY, l = 0.f;  // head l16; l: the tokens of this lane's quad
+  float acc[kG][kE];              // columns l16 * kE + e over the tokens of this lane's quad
+#pragma unroll
+  for (int g = 0; g < kG; ++g)
+#pragma unroll
+    for (int e = 0; e < kE; ++e) acc[g][e] = 0.f;
+  __syncthreads();  // page rows staged
+
+  // Page rows of this wave's batches j0 .. j0 + 63, one per lane (-1: past the
+  // segment or outside the pool).  A page holds a multiple of 16 tokens, so a
+  // batch lies in one page and its row is uniform.
+  int lane_row = -1;
+  auto rows_from = [&](int j0) {
+    const int t = (wave + kWaves * (j0 + lane)) * kTok;
+    lane_row = -1;
+    if (t < T_tok) {
+      const int pg = a.p_shift >= 0 ? t >> a.p_shift : t / P;
+      if (staged) {
+        lane_row = s_rows[pg];
+      } else {
+        const int r = a.indices[sp.start + pg];
+        lane_row = (r >= 0 && r < a.rows) ? r : -1;
+      }
+    }
+  };
+  struct Batch {
+    vtx::U4 k[kSteps];
+    VRow<kE> v[4];
+    int tokens;  // of the 16, how many the segment has
+  };
+  // batch j of this wave: tokens (wave + kWaves * j) * 16 ..  (j in order).
+  // All 16 rows are loaded, of the pool's first page for a batch without one
+  // (valid addresses: every page has its P >= 16 rows), and masked off.
+  auto load = [&](int j, Batch& b) {
+    if (j % vtx::kWave == 0) rows_from(j);  // uniform
+    const int row = __builtin_amdgcn_readlane(lane_row, j % vtx::kWave);
+    const int t0 = (wave + kWaves * j) * kTok;
+    const int slot = a.p_shift >= 0 ? t0 & (P - 1) : t0 % P;
+    b.tokens = row >= 0 ? min(kTok, T_tok - t0) : 0;
+    const long long base = row >= 0 ? ((long long)row * P + slot) * kD : 0;
+    const uint16_t* kp = a.k + base + (l16 * kD + quad * 8);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) b.k[s] = vtx::ld16_stream(kp + s * 32);
+    const uint16_t* vp = a.v + base + (4 * quad * kD + l16 * kE);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) b.v[r] = load_v<kE>(vp + r * kD);
+  };
+  auto compute = [&](Batch& b) {
+    f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s)
+      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b.k[s]),
+                                                  __builtin_bit_cast(bf16x8, qf[s]), c, 0, 0, 0);
+    float p[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = 4 * quad + r < b.tokens ? c[r] * a.scale : -INFINITY;
+    // online softmax: the running max of head l16 covers every token the wave has seen
+    float bm = fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3]));
+    bm = fmaxf(bm, vtx::xshfl(bm, 16));
+    bm = fmaxf(bm, vtx::xshfl(bm, 32));
+    const float nm = fmaxf(mx, bm);
+    if (__ballot(nm > mx && l16 < G)) {  // uniform: a head's maximum grew
+      const float f = nm == -INFINITY ? 1.f : __expf(mx - nm);
+      l *= f;
+#pragma unroll
+      for (int g = 0; g < kG; ++g) {
+        const float fg = row_broadcast<kG>(f, g);
+#pragma unroll
+        for (int e = 0; e < kE; ++e) acc[g][e] *= fg;
+      }
+      mx = nm;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = mx == -INFINITY ? 0.f : __expf(p[r] - mx);  // 0 for masked tokens
+    l += (p[0] + p[1]) + (p[2] + p[3]);
+    if (b.tokens < kTok) {  // uniform: rows past the segment may hold anything, NaN too
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int w = 0; w < kE / 2; ++w) b.v[r].w[w] = 4 * quad + r < b.tokens ? b.v[r].w[w] : 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float vf[kE];
+#pragma unroll
+      for (int w = 0; w < kE / 2; ++w) {
+        vf[2 * w] = vtx::bf16_lo(b.v[r].w[w]);
+        vf[2 * w + 1] = vtx::bf16_hi(b.v[r].w[w]);
+      }
+#pragma unroll
+      for (int g = 0; g < kG; ++g) {
+        const float pg = row_broadcast<kG>(p[r], g);
+#pragma unroll
+        for (int e = 0; e < kE; ++e) acc[g][e] = fmaf(pg, vf[e], acc[g][e]);
+      }
+    }
+  };
+  // two register buffers, as in paged_decode_attention_kernel
+  const int batches = (T_tok + kTok - 1) / kTok;
+  const int nb = batches > wave ? (batches - wave + kWaves - 1) / kWaves : 0;
+  if (nb > 0) {  // uniform over the wave
+    Batch ba, bb;
+    load(0, ba);
+    for (int j = 0; j < nb; j += 2) {
+      load(j + 1, bb);
+      compute(ba);
+      load(j + 2, ba);
+      if (j + 1 < nb) compute(bb);
+    }
+  }
+
+  // fold the quads of the wave, then the waves
+#pragma unroll
+  for (int d = 16; d < vtx::kWave; d <<= 1) {
+    l += vtx::xshfl(l, d);
+#pragma unroll
+    for (int g = 0; g < kG; ++g)
+#pragma unroll
+      for (int e = 0; e < kE; ++e) acc[g][e] += vtx::xshfl(acc[g][e], d);
+  }
+  if (lane < kG) {
+    s_m[wave][lane] = mx;
+    s_l[wave][lane] = l;
+  }
+  if (quad == 0) {
+#pragma unroll
+    for (int g = 0; g < kG; ++g)
+#pragma unroll
+      for (int e = 0; e < kE; ++e) s_acc[wave][g][l16 * kE + e] = acc[g][e];
+  }
+  __syncthreads();
+  attn_merge<kWaves, kG, kD, kSplit, T>(a, sp, s_m, s_l, s_acc);
 }
 
 // Outputs of the split segments: one workgroup per (segment, query head)
@@ -441,24 +715,32 @@ __global__ __launch_bounds__(kCombineWaves * vtx::kWave) void attention_combine_
   }
 }
 
-template <int LPR, int VPL, int kG>
-void launch_one(const AttnArgs& a, hipStream_t s) {
+// Three and more heads of 64 or 128 columns in pages of a multiple of 16 tokens
+// take the matrix cores' kernel (why: there), the rest the VALU's.
+template <int kD, int kG>
+int launch_one(const AttnArgs& a, hipStream_t s) {
+  constexpr int LPR = kD == 64 ? 8 : 16, VPL = kD / (LPR * 8);
   constexpr int T = attn_threads<LPR, VPL, kG>();
-  if (a.nsplit == 1) {
-    paged_decode_attention_kernel<LPR, VPL, kG, false><<<a.segments, T, 0, s>>>(a);
-    return;
+  const bool split = a.nsplit > 1;
+  const int grid = a.segments * a.nsplit;
+  bool matrix = false;
+  if constexpr (kD <= 128 && kG >= 4) {
+    matrix = a.P % 16 == 0;
+    if (matrix && split) decode_attention_mfma_kernel<kD, kG, true><<<grid, kMfmaThreads, 0, s>>>(a);
+    else if (matrix) decode_attention_mfma_kernel<kD, kG, false><<<grid, kMfmaThreads, 0, s>>>(a);
   }
-  paged_decode_attention_kernel<LPR, VPL, kG, true><<<a.segments * a.nsplit, T, 0, s>>>(a);
-  attention_combine_kernel<LPR * VPL * 8><<<a.segments * a.G, kCombineWaves * vtx::kWave, 0, s>>>(a);
+  if (!matrix && split) paged_decode_attention_kernel<LPR, VPL, kG, true><<<grid, T, 0, s>>>(a);
+  else if (!matrix) paged_decode_attention_kernel<LPR, VPL, kG, false><<<grid, T, 0, s>>>(a);
+  if (split) attention_combine_kernel<kD><<<a.segments * a.G, kCombineWaves * vtx::kWave, 0, s>>>(a);
+  return vtx::check_launch("paged_decode_attention");
 }
 
-template <int LPR, int VPL>
+template <int kD>
 int launch_g(const AttnArgs& a, hipStream_t s) {
-  if (a.G <= 1) launch_one<LPR, VPL, 1>(a, s);
-  else if (a.G <= 2) launch_one<LPR, VPL, 2>(a, s);
-  else if (a.G <= 4) launch_one<LPR, VPL, 4>(a, s);
-  else launch_one<LPR, VPL, 8>(a, s);
-  return vtx::check_launch("paged_decode_attention");
+  if (a.G <= 1) return launch_one<kD, 1>(a, s);
+  if (a.G <= 2) return launch_one<kD, 2>(a, s);
+  if (a.G <= 4) return launch_one<kD, 4>(a, s);
+  return launch_one<kD, 8>(a, s);
 }
 
 }  // namespace
@@ -554,9 +836,9 @@ int attention_impl(const char* what, const uint16_t* q, uint16_t* o, const uint1
   }
   hipStream_t s = vtx::as_stream(stream);
   switch (head_dim) {
-    case 64: return launch_g<8, 1>(a, s);
-    case 128: return launch_g<16, 1>(a, s);
-    default: return launch_g<16, 2>(a, s);
+    case 64: return launch_g<64>(a, s);
+    case 128: return launch_g<128>(a, s);
+    default: return launch_g<256>(a, s);
   }
 }
 
