@@ -777,12 +777,12 @@ def test_sparse_attention_equals_dense_when_budget_covers_all(gpu):
 # requests beside long ones, many segments of uneven and of equal lengths
 _SPLIT_TABLES = {
     "edge": ([2048, 2049, 2047], 1, 16, 2, 128),
-    "empty": ([0, 5000, 1, 700, 0], 2, 4, 1, 64),
+    "empty": ([0, 9000, 1, 2700, 0], 2, 4, 1, 64),
     "page1": ([3001], 2, 1, 4, 128),
     "wide": ([1800, 33], 2, 32, 3, 256),
     "heads8": ([6000, 16], 4, 64, 8, 128),
-    "uneven": ([9000, 300, 4100] + [1900 + 37 * i for i in range(15)], 8, 16, 2, 64),
-    "equal": ([2100] * 16, 8, 16, 2, 64),
+    "uneven": ([14000, 300, 7100] + [2900 + 37 * i for i in range(15)], 8, 16, 2, 128),
+    "equal": ([2100] * 16, 8, 16, 4, 64),
 }
 
 

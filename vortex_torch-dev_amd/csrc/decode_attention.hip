@@ -757,26 +757,44 @@ struct SplitPlan {
   int32_t nsplit, cus, min_avg_tokens, ragged_only;
 };
 
-// Fewer than half a segment per CU leave the chip idle, so splitting pays
-// from about 500 tokens on (8 segments: 512 tokens 11.5 -> 10.7 us, 2048
-// tokens 31.4 -> 11.4; 64 segments: 768 tokens 15.2 -> 14.7, 1024 tokens
-// 19.2 -> 16.5; the line 384 + 8 tokens per segment keeps 32 segments of 512,
-// 11.8 against 12.7, whole).  With more segments a table gains by evening out
-// its lengths (128 segments of 1k to 16k tokens: 219 -> 108 us; 256 of 0.5k to
-// 8k: 128 -> 109), and one of equal lengths only pays for the combine launch
-// (128 of 2048: 32.3 us, 34.2 with it; 256: 46.6 and 48.8), so from a segment
-// per CU on, where an uneven table gains least, the line lies at 4096.
-SplitPlan split_plan(long long segments, long long indices_len, int32_t page_size) {
+// Fewer than half a segment per CU leave the chip idle: splitting pays where a
+// whole segment takes longer than the extra workgroups and the combine launch.
+// A whole segment's time per token follows its dot products and its rows: with
+// one and two heads 5.5 us + D / 128 * (6 + 4 G) us per 1024 tokens, and a split
+// table of S segments takes about 11 to 17 us, so the line lies at 512 + 8 S
+// tokens for two heads of 128 columns and in that proportion for the others.
+// Whole / split, 8 segments: D 128, 2 heads 13.2 / 12.1 us at 544 tokens, 21.1 /
+// 12.3 at 1056; 1 head 10.6 / 11.2 and 15.9 / 11.1; D 64, 1 head 8.4 / 10.5,
+// 10.8 / 10.6 and (2112) 15.9 / 11.1.  16 segments: D 64, 1 head 8.6 / 13.3, 10.9
+// / 14.0 and 16.3 / 15.1.  52 of 1024 tokens: D 64, 1 head 11.0 / 16.0; D 128 16.8
+// / 17.5.  Three and more heads (4 heads, 52 segments of 1024: 40.5 whole on the
+// VALU, 17.8) and rows of 256 columns split from 384 + 8 S tokens on.  With more segments a table gains by evening out its lengths
+// (128 segments of 1k to 16k tokens: 219 -> 108 us; 256 of 0.5k to 8k: 128 ->
+// 109), and one of equal lengths only pays for the combine launch (128 of 2048:
+// 32.3 us, 34.2 with it; 240 of 2048, 1 head: 42.4 and 44.5, D 64 24.3 and 26.7),
+// so the line lies where that is a few percent.
+SplitPlan split_plan(long long segments, long long indices_len, int32_t page_size, int32_t group_size,
+                     int32_t head_dim) {
   const int cus = vtx::device_cu_count();
   SplitPlan p{1, 1, 0, 0};
   if (cus <= 0 || segments <= 0 || segments >= kMaxSplitSegmentsPerCu * (long long)cus) return p;
   p.cus = cus;
   p.ragged_only = 2 * segments >= cus;
-  p.min_avg_tokens = !p.ragged_only ? (int32_t)(384 + 8 * segments) : (segments < cus ? 2048 : 4096);
+  const bool narrow = group_size <= 2 && head_dim <= 128;
+  long long least = !p.ragged_only ? (narrow ? 512 : 384) + 8 * segments
+                                   : (segments >= cus ? 4096 : (narrow ? 3072 : 2048));
+  if (narrow) least = least * 896 / (head_dim * (3 + 2 * group_size));  // (1 for two heads of 128 columns)
+  p.min_avg_tokens = (int32_t)least;
   // (a table that cannot hold this average is not split whatever it holds)
-  if (indices_len * page_size < (long long)p.min_avg_tokens * segments) return p;
-  const long long n = (8LL * cus + segments - 1) / segments;
-  p.nsplit = (int32_t)(n > kMaxSplit ? kMaxSplit : n);
+  if (indices_len * page_size < least * segments) return p;
+  // chunks of a segment: as many as even out the longest, and no more than a
+  // table of this capacity can need (chunks_of cuts no chunk below its minimum
+  // but the last, so this bound changes no table's chunks)
+  const long long min_pages = (kMinChunkTokens + page_size - 1) / page_size;
+  long long n = (8LL * cus + segments - 1) / segments;
+  n = n > kMaxSplit ? kMaxSplit : n;
+  const long long need = (indices_len + min_pages - 1) / min_pages;
+  p.nsplit = (int32_t)(n > need ? need : n);
   return p;
 }
 
@@ -820,7 +838,7 @@ int attention_impl(const char* what, const uint16_t* q, uint16_t* o, const uint1
   a.ml = nullptr;
   a.acc = nullptr;
   if (workspace) {
-    const SplitPlan p = split_plan(segments, kv_indices_len, page_size);
+    const SplitPlan p = split_plan(segments, kv_indices_len, page_size, group_size, head_dim);
     const long long rows = segments * p.nsplit * group_size;
     if (p.nsplit > 1) {
       if (workspace_len < rows * (head_dim + 2) || !vtx::aligned16(workspace))
@@ -863,7 +881,7 @@ extern "C" int64_t vtx_paged_decode_attention_workspace_len(int32_t batch_size, 
       !vtx_paged_decode_attention_supported(head_dim, group_size))
     return 0;
   const long long segments = (long long)batch_size * num_kv_heads;
-  const SplitPlan p = split_plan(segments, kv_indices_len, page_size);
+  const SplitPlan p = split_plan(segments, kv_indices_len, page_size, group_size, head_dim);
   return p.nsplit > 1 ? segments * p.nsplit * group_size * (head_dim + 2) : 0;
 }
 
