@@ -159,7 +159,9 @@ def fused_kernel_name(batch: W.DecodeBatch) -> str:
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     layout = fused_layout()
     mp = batch.max_pages_per_request
-    auto = segments < 2 * cus if batch.head_dim >= 256 else mp > 512 and 3 * segments < 2 * cus
+    auto = segments < 2 * cus if batch.head_dim >= 256 else mp > 512 and (
+        3 * segments < 2 * cus or (batch.head_dim == 128 and batch.topk <= 64 and segments * -(-mp // 256) <= 4 * cus
+                                   and (segments > cus or batch.topk > 32)))
     if layout == 2 or (layout == 0 and auto):
         # the library's split_threads / split_pass / chunk choice, with the
         # topK op's workspace (staging zone present)

@@ -216,7 +216,9 @@ int vtx_topk_select(const uint16_t* score, int64_t score_len,
  * (with the counters given, split where few segments would leave compute units
  * idle for longer than a split segment's hand-off takes: head_dim >= 256 and
  * fewer than two segments per compute unit, or head_dim <= 128, over 512 pages
- * and fewer than two for three units), VTX_FUSED_SEGMENT or VTX_FUSED_SPLIT.  Outputs are
+ * and fewer than two for three units, or head_dim 128, over 512 pages, small
+ * chunks that fit the device at once and more than one segment per unit or
+ * 32 kept pages), VTX_FUSED_SEGMENT or VTX_FUSED_SPLIT.  Outputs are
  * identical in every mode.
  *
  * schedule (optional, NULL for none): the fused_schedule vtx_plan_decode

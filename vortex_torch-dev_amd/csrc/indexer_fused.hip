@@ -1253,9 +1253,21 @@ int split_chunk(int dim, bool large, bool quad) {
 // pages 7.0 / 9.0 us, 64 of 512 10.3 / 10.6 (top-64), 256 of 512 9.8 / 11.9,
 // 256 of 1024 15.0 / 17.1, 256 of 2048 25.0 / 28.2; 8 of 1024 pages 12.2 /
 // 9.8, 64 of 1024 12.4 / 10.7, 128 of 1024 12.9 / 12.2, 64 of 2048 24 / 14.
-bool split_pays(long long segments, long long max_pages, int dim, int cus) {
+//
+// Rows of 128 columns whose small chunks of four waves (split_chunk) are all
+// on the chip at once also pay where whole segments are at their slowest: past
+// a segment per CU, whose second round of 8-wave workgroups is nearly empty
+// (304 of 600 equal pages 21.6 / 18.7 us, of 760 23.1 / 20.7; 1024, which no
+// longer fit, 26.9 / 31.3), and with more than 32 kept pages, whose select
+// takes a 16-wave workgroup longer (208 of 600, top-64 17.2 / 16.4, top-30 15.2
+// / 16.3; 208 of 1500, which do not fit, 26.7 / 32.1).
+bool split_pays(long long segments, long long max_pages, int dim, int topk, int cus) {
   if (dim >= 256) return segments < 2LL * cus;
-  return max_pages > 512 && 3 * segments < 2LL * cus;
+  if (max_pages <= 512) return false;
+  const long long chunk = split_chunk(dim, false, true);
+  const bool fits = dim == 128 && topk <= vtx::kMaxBitonicRunK && segments <= kStageMaxSegments &&
+                    segments * ((max_pages + chunk - 1) / chunk) <= 4LL * cus;
+  return 3 * segments < 2LL * cus || (fits && (segments > cus || topk > 32));
 }
 
 // blocks: the grid, xcd: work ids per XCD (8 * xcd workgroups take work
@@ -1464,7 +1476,7 @@ int fused_impl(const uint16_t* q, int64_t q_rows, int32_t group_size, const uint
   if (cus <= 0) return vtx::fail(VTX_E_DEVICE, "indexer_fused: cannot query the compute unit count");
 
   const bool split = mode == VTX_FUSED_SPLIT ||
-                     (mode == VTX_FUSED_AUTO && have_counters && split_pays(eff_batch_size, want, head_dim, cus));
+                     (mode == VTX_FUSED_AUTO && have_counters && split_pays(eff_batch_size, want, head_dim, a.topk, cus));
   // The CMean runs inside the launch for decode-sized loc and a 16-byte
   // aligned K pool: in the segment layout for rows of one 16-byte vector per
   // lane (its tile layout is then the scoring layout), in the split layout
