@@ -146,28 +146,29 @@ def test_fused_segment_and_split_layouts_agree(gpu, name, cmean):
         assert (out[_hip.FUSED_SPLIT][0] != _bits(y0)).any() or int(((loc + 1) % P == 0).sum()) == 0
 
 
+@pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("topk", [30, 40])
 @pytest.mark.parametrize("batch_size,pages", [(1, 256), (3, 257), (2, 512), (2, 513), (2, 1024), (2, 1025),
                                               (33, 513), (33, 1025)])
-def test_fused_auto_layout_equals_the_others(gpu, batch_size, pages, topk):
+def test_fused_auto_layout_equals_the_others(gpu, batch_size, pages, topk, D):
     """At the page and segment counts where FUSED_AUTO changes its layout or
     its workgroup size (264 segments: over one per compute unit of 256), it
     writes the bits of the segment and the split layout, with the CMean."""
     dev = gpu
     lens = [pages * 2] + [max(2, (pages - 7 * i) * 2 - i % 2) for i in range(1, batch_size)]
     batch = W.make_batch(lens, pool_pages=sum((n + 1) // 2 for n in lens) + 3, seed=51, page_size=2, num_kv_heads=8,
-                         group_size=2, head_dim=64, topk=topk, eos=0)
+                         group_size=2, head_dim=D, topk=topk, eos=0)
     loc = W.decode_loc(batch).to(dev)
     ic, _ = W.make_contexts(batch, dev)
     _plan(batch, ic, dev)
     S, rows = batch.batch * 8, batch.pool_pages * 8
-    q = _wide_q((S, 2, 64), 11, dev)
-    k = W.randn_bf16((rows, 2, 64), 3, dev)
-    y0 = W.randn_bf16((rows, 1, 64), 2, dev, std=0.25)
+    q = _wide_q((S, 2, D), 11, dev)
+    k = W.randn_bf16((rows, 2, D), 3, dev)
+    y0 = W.randn_bf16((rows, 1, D), 2, dev, std=0.25)
     out = {}
     for mode in (_hip.FUSED_AUTO, _hip.FUSED_SEGMENT, _hip.FUSED_SPLIT):
         y, sp = y0.clone(), ic.sparse_kv_indices.clone()
-        qm = torch.full((S, 1, 64), 3.0, device=dev, dtype=torch.bfloat16)
+        qm = torch.full((S, 1, D), 3.0, device=dev, dtype=torch.bfloat16)
         sc = torch.full((ic.dense_kv_indices.numel(), 1, 1), -5.0, device=dev, dtype=torch.bfloat16)
         counters = torch.zeros(_hip.indexer_fused_workspace_len(S), dtype=torch.int32, device=dev)
         _hip.indexer_fused(q, qm, y, sc, ic.dense_kv_indptr, ic.sparse_kv_indptr, ic.dense_kv_indices, sp, S, topk,
