@@ -859,3 +859,55 @@ def test_decode_attention_many_heads(gpu, name, G, D):
             v[rows:rows + H, n % P:] = float("inf")
     o = paged_decode_attention(q, k, v, *args, len(lens), H)
     np.testing.assert_allclose(_f(_bits(o)), _f(exp), rtol=2 ** -7, atol=1e-4)
+
+
+def _hand_table(lens, P, gpu, seed, outside=False):
+    """A block table over pool rows 1 .. (row 0 is nobody's), and the same table
+    without the entries that `outside` puts outside the pool."""
+    n = [(x + P - 1) // P for x in lens]
+    rows = sum(n) + 1
+    perm = torch.randperm(rows - 1, generator=torch.Generator().manual_seed(seed)) + 1
+    ip, idx, kept_ip, kept = [0], [], [0], []
+    for c in n:
+        seg = perm[ip[-1]:ip[-1] + c].tolist()
+        bad = [outside and i % 3 == 1 and i < c - 1 for i in range(c)]
+        idx += [(-1 if i % 2 else rows) if b else r for i, (r, b) in enumerate(zip(seg, bad))]
+        kept += [r for r, b in zip(seg, bad) if not b]
+        ip.append(len(idx))
+        kept_ip.append(len(kept))
+    last = [(x - 1) % P + 1 if x else 0 for x in lens]
+    dev = [torch.tensor(t, dtype=torch.int32, device=gpu) for t in (ip, idx, last)]
+    return rows, dev, [np.asarray(t, np.int32) for t in (kept_ip, kept, last)]
+
+
+def _attend_whole(q, k, v, ip, idx, last, S, G, D, P):
+    """The C entry that splits no segment and needs no workspace."""
+    o = torch.empty_like(q)
+    rc = _hip.load_library().vtx_paged_decode_attention(
+        q.data_ptr(), o.data_ptr(), k.data_ptr(), v.data_ptr(), k.shape[0], ip.data_ptr(), idx.data_ptr(),
+        idx.numel(), last.data_ptr(), S, 1, G, D, P, 1.0 / np.sqrt(D), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    return o
+
+
+@pytest.mark.parametrize("outside", [False, True])
+@pytest.mark.parametrize("lens", [[1, 15, 33, 0, 700], [2101, 1999, 2500]])
+@pytest.mark.parametrize("G,D,P", [(1, 64, 16), (2, 64, 16), (1, 128, 16), (2, 128, 16), (2, 256, 16), (5, 256, 16),
+                                   (4, 128, 8), (8, 64, 24), (4, 128, 16)])
+def test_decode_attention_ignores_rows_of_others(gpu, G, D, P, lens, outside):
+    """Pool rows that no segment holds may be NaN and infinities, the first row
+    (which masked tokens load) too: whole and split, in both kernels, with and
+    without entries outside the pool, the result is the oracle's over the
+    entries inside (within its bf16 rounding)."""
+    from vortex_torch.decode_attention import paged_decode_attention
+
+    rows, (ip, idx, last), kept = _hand_table(lens, P, gpu, 5, outside)
+    k = W.randn_bf16((rows, P, D), 23, gpu)
+    v = W.randn_bf16((rows, P, D), 24, gpu)
+    q = W.randn_bf16((len(lens) * G, D), 25, gpu)
+    exp = _f(O.paged_decode_attention(_bits(q), _bits(k), _bits(v), *kept, len(lens), 1, 1.0 / np.sqrt(D)))
+    k[0], v[0] = float("nan"), float("inf")
+    v[0, ::2] = float("nan")
+    for o in (paged_decode_attention(q, k, v, ip, idx, last, len(lens), 1),
+              _attend_whole(q, k, v, ip, idx, last, len(lens), G, D, P)):
+        np.testing.assert_allclose(_f(_bits(o)), exp, rtol=2 ** -7, atol=1e-4)

@@ -276,7 +276,8 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
   const int nb = batches > wave ? (batches - wave + kWaves - 1) / kWaves : 0;
 
   // K and V of batch j; tokens past the segment or on rows outside the pool
-  // load the pool's first row (a valid address) and are masked off
+  // load the pool's first row (a valid address) and are masked off, its values
+  // with them: they may be anything, NaN and infinities too
   auto load = [&](int j, vtx::U4 (&kv)[kB][VPL], vtx::U4 (&vv)[kB][VPL], bool (&ok)[kB]) {
 #pragma unroll
     for (int i = 0; i < kB; ++i) {
@@ -301,7 +302,18 @@ __global__ __launch_bounds__((attn_threads<LPR, VPL, kG>()),
       }
     }
   };
-  auto compute = [&](const vtx::U4 (&kv)[kB][VPL], const vtx::U4 (&vv)[kB][VPL], const bool (&ok)[kB]) {
+  auto compute = [&](const vtx::U4 (&kv)[kB][VPL], vtx::U4 (&vv)[kB][VPL], const bool (&ok)[kB]) {
+    bool live = true;
+#pragma unroll
+    for (int i = 0; i < kB; ++i) live = live && ok[i];
+    if (__ballot(!live)) {  // uniform: few batches (a segment's last, rows outside the pool)
+#pragma unroll
+      for (int i = 0; i < kB; ++i)
+#pragma unroll
+        for (int v = 0; v < VPL; ++v)
+          vv[i][v] = vtx::U4{ok[i] ? vv[i][v].x : 0u, ok[i] ? vv[i][v].y : 0u, ok[i] ? vv[i][v].z : 0u,
+                             ok[i] ? vv[i][v].w : 0u};
+    }
     // scores: every lane of a token's LPR group ends with the full dot
     float sc[kB][kG];
 #pragma unroll
