@@ -476,6 +476,16 @@ int vtx_page_reduce_multi(const uint16_t* x, int64_t x_rows,
                           const int64_t* loc, int64_t nnz, int32_t num_kv_heads,
                           int32_t page_size, int32_t dim, void* stream);
 
+/*
+ * How a dim-1 reduction of nnz > 0 loc entries, on 16-byte aligned buffers,
+ * deals the tiles that a block of 256 entries closes: to *share workgroups,
+ * whose four waves take *per_round tiles at a time each.  No launch, no device
+ * needed.
+ */
+int vtx_page_reduce_sharing(int32_t rows_per_tile, int32_t cols, int32_t n_out, const int32_t* reduce_types,
+                            int64_t nnz, int32_t num_kv_heads, int32_t page_size, int32_t* share,
+                            int32_t* per_round);
+
 /* ------------------------------------------------------------------------
  * Workload-walking indexer ops (GeMM, elementwise, reductions, segment
  * softmax / normalize): the ops of the GQA and Quest flows.

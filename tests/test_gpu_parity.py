@@ -409,3 +409,27 @@ def test_reduce_burst_equals_small_calls(gpu, nnz, heads, page, cols):
         _hip.page_reduce_multi(k, parts, types, loc[at:at + 256].contiguous(), heads, page)
     for a, b in zip(whole, parts):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("types", [[O.MAX, O.MIN], [O.MEAN, O.MAX, O.MIN, O.L2NORM], [O.MIN]])
+@pytest.mark.parametrize("nnz", [300, 1024, 9001, 70000])
+@pytest.mark.parametrize("heads,page,cols", [(8, 16, 128), (1, 16, 64), (1, 512, 128), (3, 8, 64), (8, 2, 256),
+                                             (2, 256, 576), (1, 16, 512)])
+def test_reduce_shared_tiles_equal_small_calls(gpu, heads, page, cols, nnz, types):
+    """As above for CMax + CMin, for all four statistics and for one, at the
+    grid sizes where the workgroups per block of entries and the tiles per wave
+    change, with pages wider than a block too."""
+    pool = 300 + nnz // page
+    g = torch.Generator().manual_seed(nnz + heads)
+    loc = torch.randperm(pool * page, generator=g)[:nnz]
+    n = loc.numel()
+    loc[:n // 16] = torch.randperm(pool, generator=g)[torch.arange(n // 16) % pool] * page + page - 1
+    loc = loc.to(gpu)
+    k = W.randn_bf16((pool * heads, page, cols), 5, gpu)
+    whole, parts = ([torch.full((pool * heads, 1, cols), -3.0, dtype=torch.bfloat16, device=gpu) for _ in types]
+                    for _ in range(2))
+    _hip.page_reduce_multi(k, whole, types, loc, heads, page)
+    for at in range(0, n, 256):
+        _hip.page_reduce_multi(k, parts, types, loc[at:at + 256].contiguous(), heads, page)
+    for a, b in zip(whole, parts):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))

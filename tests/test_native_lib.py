@@ -51,6 +51,35 @@ def test_host_side_argument_errors():
     assert lib.vtx_indexer_fused_supported(128) == 1 and lib.vtx_indexer_fused_supported(100) == 0
 
 
+@pytest.mark.parametrize("types", [[_hip.REDUCE_MEAN], [_hip.REDUCE_MEAN, _hip.REDUCE_MAX],
+                                   [_hip.REDUCE_MAX, _hip.REDUCE_MIN],
+                                   [_hip.REDUCE_MEAN, _hip.REDUCE_MAX, _hip.REDUCE_MIN, _hip.REDUCE_L2NORM]])
+@pytest.mark.parametrize("cols", [64, 128, 256, 512, 576])
+def test_page_reduce_sharing_leaves_no_wave_a_queue(cols, types):
+    """The workgroups that share a block of 256 loc entries take the tiles it
+    closes in one round of what their waves really do at a time (several tiles
+    only where the instance's registers fit), or there are sixteen; and sixteen
+    while the grid is small, also where a whole page is wider than a block."""
+    lib = _hip.load_library()
+    rt = (ctypes.c_int32 * len(types))(*types)
+    # statistics that the instance accumulates, times the levels of its fold over a wave's row groups
+    stats = len(types) if types != [_hip.REDUCE_MAX, _hip.REDUCE_MIN] else 4
+    lpr = cols // 8
+    fits = lpr <= 64 and 64 % lpr == 0 and {8: 4, 16: 3, 32: 2, 64: 1}[lpr] * stats <= 8
+    for page in (1, 8, 16, 17, 32, 256, 512):
+        for heads in (1, 2, 3, 8):
+            for nnz in (1, 256, 768, 769, 1024, 1025, 4096, 8192, 8193, 65536, 1 << 20):
+                share, per = ctypes.c_int32(), ctypes.c_int32()
+                assert lib.vtx_page_reduce_sharing(page, cols, len(types), rt, nnz, heads, page, share, per) == 0
+                what = (page, heads, nnz, share.value, per.value)
+                tiles, blocks = max(1, 256 // page) * heads, -(-nnz // 256)
+                assert 1 <= share.value <= 16, what
+                assert per.value == 1 or (per.value == 64 // lpr and fits and page <= 16 and blocks >= 4), what
+                assert share.value == 16 or share.value * 4 * per.value >= tiles, what
+                if blocks <= 32:
+                    assert share.value == 16, what
+
+
 def test_missing_library_fails_loudly(tmp_path):
     with pytest.raises(RuntimeError, match="not found"):
         _hip.load_library(tmp_path / "nope.so")

@@ -21,6 +21,8 @@
 //     each lane one column vector and load 8 rows of it at a time;
 //   * one pass over the tile feeds up to four outputs (the fused entry point),
 //     so CMean + CMax read K once.
+#include <algorithm>
+
 #include "vtx_device.h"
 #include "vtx_host.h"
 #include "vtx_page_reduce.h"
@@ -51,7 +53,8 @@ __device__ __forceinline__ void store_one(const ReduceArgs& a, int o, long long 
 }
 
 constexpr int kLaneRows = 16;    // rows of the tallest tile that one lane per column vector reduces
-constexpr int kBurstBlocks = 4;  // from so many blocks of loc entries on, a burst (1024 entries and more)
+constexpr int kBurstBlocks = 4;  // from so many blocks of loc entries on, a burst (769 entries and more)
+constexpr int kMaxShare = 16;    // workgroups that share one block of entries
 
 // The pages closed by this block's 256 loc entries (the workgroups that share
 // a block of entries split its tiles by index, so they all see the same list).
@@ -59,8 +62,8 @@ __device__ __forceinline__ int collect_pages(const ReduceArgs& a, long long* fir
   return vtx::collect_pages<kThreads>(a, (long long)blockIdx.x * kThreads, first_row, wave_count);
 }
 
-// dim 1, C = 8 * LPR with LPR | 64.  Bursts of tiles of up to 16 rows (and
-// a statistic set whose registers fit): lane = (tile slot, 16-byte column
+// dim 1, C = 8 * LPR with LPR | 64.  lane_tiles (share_tiles: larger bursts of
+// tiles of up to 16 rows, of a statistic set whose registers fit): lane = (tile slot, 16-byte column
 // vector), a wave takes 64 / LPR tiles at once and each lane reduces all rows
 // of its column alone (vtx::tile_stats_lane), so all of a tile's rows are in
 // flight together, nothing crosses lanes and every lane writes its own
@@ -68,7 +71,7 @@ __device__ __forceinline__ int collect_pages(const ReduceArgs& a, long long* fir
 // folded by an xor tree (vtx::tile_stats_vec).  Both give the same bits.
 // NEED: statistics to accumulate (kNeed* mask covering every output's type).
 template <int LPR, int NEED>
-__global__ __launch_bounds__(kThreads) void reduce_rows_vec_kernel(ReduceArgs a) {
+__global__ __launch_bounds__(kThreads) void reduce_rows_vec_kernel(ReduceArgs a, int lane_tiles) {
   __shared__ long long first_row[kThreads];
   __shared__ int wave_count[kWavesPerBlock];
   const int pages = collect_pages(a, first_row, wave_count);
@@ -79,10 +82,10 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_vec_kernel(ReduceArgs a)
   const int R = a.rows_per_tile;
   const int tiles = pages * a.heads;
 
-  if constexpr (vtx::lane_tiles_fit<LPR, NEED>()) {
-    // (a decode-sized loc, whose few tiles are spread over several
-    // workgroups, keeps one tile per wave: more waves share the latency)
-    if (R <= kLaneRows && gridDim.x >= kBurstBlocks) {  // uniform
+  if constexpr (vtx::lane_tiles_fit(LPR, NEED)) {
+    // uniform (lane_tiles implies the bound; without it here the compiler adds
+    // the rows up more slowly: 59,576 entries, 8 heads 29.8 us instead of 28.8)
+    if (R <= kLaneRows && lane_tiles) {
       constexpr int kSlots = vtx::kWave / LPR;  // tiles per wave at once; lane group grp takes slot grp
       for (int t0 = (blockIdx.y * kWavesPerBlock + wave) * kSlots; t0 < tiles;
            t0 += gridDim.y * kWavesPerBlock * kSlots) {
@@ -212,18 +215,72 @@ __global__ __launch_bounds__(kThreads) void reduce_generic_kernel(ReduceArgs a, 
 
 // Single reductions and CMean + CMax get their own code; other mixes
 // accumulate every statistic.
+constexpr int instance_need(int need) {
+  return need == kNeedSum || need == kNeedMax || need == kNeedMin || need == kNeedSq || need == (kNeedSum | kNeedMax)
+             ? need
+             : kNeedAll;
+}
+
 template <int LPR>
-void launch_vec(const ReduceArgs& a, int need, dim3 grid, hipStream_t s) {
-  switch (need) {
-    case kNeedSum: reduce_rows_vec_kernel<LPR, kNeedSum><<<grid, kThreads, 0, s>>>(a); break;
-    case kNeedMax: reduce_rows_vec_kernel<LPR, kNeedMax><<<grid, kThreads, 0, s>>>(a); break;
-    case kNeedMin: reduce_rows_vec_kernel<LPR, kNeedMin><<<grid, kThreads, 0, s>>>(a); break;
-    case kNeedSq: reduce_rows_vec_kernel<LPR, kNeedSq><<<grid, kThreads, 0, s>>>(a); break;
+void launch_vec(const ReduceArgs& a, int need, dim3 grid, int lane_tiles, hipStream_t s) {
+  switch (instance_need(need)) {
+    case kNeedSum: reduce_rows_vec_kernel<LPR, kNeedSum><<<grid, kThreads, 0, s>>>(a, lane_tiles); break;
+    case kNeedMax: reduce_rows_vec_kernel<LPR, kNeedMax><<<grid, kThreads, 0, s>>>(a, lane_tiles); break;
+    case kNeedMin: reduce_rows_vec_kernel<LPR, kNeedMin><<<grid, kThreads, 0, s>>>(a, lane_tiles); break;
+    case kNeedSq: reduce_rows_vec_kernel<LPR, kNeedSq><<<grid, kThreads, 0, s>>>(a, lane_tiles); break;
     case kNeedSum | kNeedMax:
-      reduce_rows_vec_kernel<LPR, kNeedSum | kNeedMax><<<grid, kThreads, 0, s>>>(a);
+      reduce_rows_vec_kernel<LPR, kNeedSum | kNeedMax><<<grid, kThreads, 0, s>>>(a, lane_tiles);
       break;
-    default: reduce_rows_vec_kernel<LPR, kNeedAll><<<grid, kThreads, 0, s>>>(a); break;
+    default: reduce_rows_vec_kernel<LPR, kNeedAll><<<grid, kThreads, 0, s>>>(a, lane_tiles); break;
   }
+}
+
+// How the closed pages' tiles of one block of entries are dealt: `share`
+// workgroups take them (each rescans the same entries), their waves
+// `per_round` tiles at a time each.
+struct Sharing {
+  long long share;
+  int per_round;
+};
+
+// vec: rows of 16-byte vectors, aligned (lpr of them); need: what the launched
+// instance accumulates.  The tiles of a block are counted as those of whole
+// pages (a decode step of as many requests closes as many on average).
+//
+// One round of the workgroups' waves takes them all, where sixteen can, so
+// that scans and first loads of some overlap the tiles of others; and while
+// the grid stays under 512 workgroups there are sixteen, so that requests
+// whose pages all close together (256 tiles per head and block) find waves:
+// they cost nothing where there is no work.  CMax + CMin (every statistic
+// accumulated, one tile per wave), 16-token pages of 128 columns, 8 heads: 32
+// blocks 42 us with 8 workgroups each, 36 with 16; 512 blocks, read from
+// memory, 247 with one and 154 with eight; 64 columns, 2 heads, 32 blocks 42
+// with one and 7.2 with 16.  Decode of 1024 requests, one head, 256-token
+// pages that all close: 739 us with one workgroup per block, 50 with 16.
+// CMean + CMax of 65,536 pages of 8 heads, lane_tiles: 514 with one, 495 with
+// four and eight.
+//
+// lane_tiles (kWave / lpr tiles per wave at once, without the fold across
+// lanes, but 16 loads per lane at once) pays where there are more tiles than
+// waves to take them one at a time: from 8192 tiles on (4096 with two
+// statistics or more, whose fold is longer), or where a block has more than
+// two rounds' (one round's) tiles.  CMean, 128 columns, one tile per wave /
+// lane tiles: 8 heads, 16 blocks 5.1 / 6.2 us, 128 blocks 15.1 / 13.1; one
+// head, 4 blocks 3.8 / 4.8, 128 blocks 4.4 / 7.1; CMean + CMax, 8 heads, 8
+// blocks 6.0 / 5.3.  256 columns and more have two tiles or one per wave, which
+// a single statistic gains nothing from (8 heads, 128 blocks 25.2 / 27.9).
+Sharing share_tiles(long long blocks, int page, int heads, int rows, bool vec, int lpr, int need) {
+  const long long tiles = (page < kThreads ? kThreads / page : 1) * (long long)heads;
+  const int stats = __builtin_popcount(need);
+  Sharing sh{1, 1};
+  if (vec && blocks >= kBurstBlocks && rows <= kLaneRows && lpr <= vtx::kWave && vtx::kWave % lpr == 0 && lpr >= 8 &&
+      vtx::lane_tiles_fit(lpr, need) && (stats > 1 || vtx::kWave / lpr > 2) &&
+      (blocks * tiles >= (stats > 1 ? 4096 : 8192) || tiles > (stats > 1 ? 1 : 2) * kMaxShare * kWavesPerBlock))
+    sh.per_round = vtx::kWave / lpr;
+  const long long round = (tiles + kWavesPerBlock * sh.per_round - 1) / (kWavesPerBlock * sh.per_round);
+  const long long few = (512 + blocks - 1) / blocks;
+  sh.share = std::min<long long>(std::max(round, few), kMaxShare);
+  return sh;
 }
 
 int launch_reduce(ReduceArgs& a, int dim, void* stream) {
@@ -257,34 +314,17 @@ int launch_reduce(ReduceArgs& a, int dim, void* stream) {
   const int lpr = a.cols / 8;
   int need = 0;
   for (int o = 0; o < a.n_out; ++o) need |= need_of(a.out_type[o]);
-  // The closed pages' tiles of one block of entries are shared by `split`
-  // workgroups (each rescans the same entries).  Few loc entries (a decode
-  // step): up to 16, so the tiles are reduced side by side rather than by 4
-  // waves.  A burst: enough that one round of a workgroup's waves takes its
-  // share of the tiles that a block of whole pages closes, so that scans and
-  // first loads of some overlap the tiles of others and the last workgroups to
-  // run are short.  65,536 pages of 8 heads, CMean + CMax: 514 us with one
-  // workgroup per block, 501 with two, 495 with four; 4,096 pages: 78 -> 34
-  // us (before, sharing also meant one tile per wave); one head (16 tiles per
-  // block), 32,768 pages: 20.7 us with one, 28 with eight.
-  long long split;
-  if (blocks < kBurstBlocks) {
-    split = 16;
-  } else {
-    const bool lane = vec && a.rows_per_tile <= kLaneRows && (lpr == 8 || lpr == 16 || lpr == 32 || lpr == 64);
-    const long long per_round = (long long)kWavesPerBlock * (lane ? vtx::kWave / lpr : 1);
-    split = (long long)kThreads / a.page * a.heads / per_round;
-    split = split < 1 ? 1 : (split > 16 ? 16 : split);
-  }
-  const dim3 grid((unsigned)blocks, (unsigned)split);
+  const Sharing sh = share_tiles(blocks, a.page, a.heads, a.rows_per_tile, vec, lpr, instance_need(need));
+  const dim3 grid((unsigned)blocks, (unsigned)sh.share);
+  const int lane_tiles = sh.per_round > 1;
   if (vec && lpr == 8) {
-    launch_vec<8>(a, need, grid, s);
+    launch_vec<8>(a, need, grid, lane_tiles, s);
   } else if (vec && lpr == 16) {
-    launch_vec<16>(a, need, grid, s);
+    launch_vec<16>(a, need, grid, lane_tiles, s);
   } else if (vec && lpr == 32) {
-    launch_vec<32>(a, need, grid, s);
+    launch_vec<32>(a, need, grid, lane_tiles, s);
   } else if (vec && lpr == 64) {
-    launch_vec<64>(a, need, grid, s);
+    launch_vec<64>(a, need, grid, lane_tiles, s);
   } else if (vec) {
     switch (need) {
       case kNeedSum: reduce_colvec_kernel<kNeedSum><<<grid, kThreads, 0, s>>>(a); break;
@@ -350,4 +390,20 @@ extern "C" int vtx_page_reduce_multi(const uint16_t* x, int64_t x_rows, int32_t 
   a.page = page_size;
   a.page_shift = vtx::log2_exact(page_size);
   return launch_reduce(a, dim, stream);
+}
+
+extern "C" int vtx_page_reduce_sharing(int32_t rows_per_tile, int32_t cols, int32_t n_out, const int32_t* reduce_types,
+                                       int64_t nnz, int32_t num_kv_heads, int32_t page_size, int32_t* share,
+                                       int32_t* per_round) {
+  vtx::clear_error();
+  if (rows_per_tile < 1 || cols < 1 || n_out < 1 || n_out > kMaxOut || !reduce_types || nnz < 1 || num_kv_heads < 1 ||
+      page_size < 1 || !share || !per_round)
+    return vtx::fail(VTX_E_INVALID, "page_reduce_sharing: bad arguments");
+  int need = 0;
+  for (int o = 0; o < n_out; ++o) need |= need_of(reduce_types[o]);
+  const Sharing sh = share_tiles((nnz + kThreads - 1) / kThreads, page_size, num_kv_heads, rows_per_tile,
+                                 cols % 8 == 0, cols / 8, instance_need(need));
+  *share = (int32_t)sh.share;
+  *per_round = sh.per_round;
+  return VTX_OK;
 }

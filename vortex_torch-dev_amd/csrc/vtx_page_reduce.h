@@ -202,11 +202,10 @@ __device__ __forceinline__ void fold_groups(const U4 (&v)[16], int R, Acc (&s)[8
 
 // Whether tile_stats_lane's registers fit for this width and statistic set
 // (16 loaded rows plus one partial per level of the group fold).
-template <int LPR, int NEED>
-__host__ __device__ constexpr bool lane_tiles_fit() {
-  constexpr int G = kWave / LPR;
-  constexpr int levels = G == 1 ? 1 : G == 2 ? 2 : G == 4 ? 3 : 4;
-  constexpr int stats = ((NEED & 1) != 0) + ((NEED & 2) != 0) + ((NEED & 4) != 0) + ((NEED & 8) != 0);
+__host__ __device__ constexpr bool lane_tiles_fit(int lpr, int need) {
+  const int groups = kWave / lpr;
+  const int levels = groups == 1 ? 1 : groups == 2 ? 2 : groups == 4 ? 3 : 4;
+  const int stats = ((need & 1) != 0) + ((need & 2) != 0) + ((need & 4) != 0) + ((need & 8) != 0);
   return levels * stats <= 8;
 }
 

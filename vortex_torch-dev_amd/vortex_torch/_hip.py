@@ -55,6 +55,10 @@ _SIGNATURES = {
         [_vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _vp],
         ctypes.c_int,
     ),
+    "vtx_page_reduce_sharing": (
+        [_i32, _i32, _i32, _vp, _i64, _i32, _i32, ctypes.POINTER(_i32), ctypes.POINTER(_i32)],
+        ctypes.c_int,
+    ),
     "vtx_indexer_fused": (
         [_vp, _i64, _i32, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64,
          _i32, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp, _i64, _vp],
