@@ -652,10 +652,13 @@ int vtx_paged_decode_attention(const uint16_t* q, uint16_t* o, const uint16_t* k
  * segment's pages may be split over several workgroups, whose partial results
  * (fp32) a second launch on the stream combines.  workspace: scratch of at
  * least vtx_paged_decode_attention_workspace_len floats, 16-byte aligned, its
- * contents neither read nor kept across calls; where that length is 0 (no
- * segment of such a table would be split) it may be NULL and the call is
- * vtx_paged_decode_attention's.  How a segment is split depends on the
- * table's contents alone, not on the buffers' capacity.
+ * contents neither read nor kept across calls.  NULL splits nothing: the call
+ * is then vtx_paged_decode_attention's (so is it where that length is 0).
+ * How a segment is split depends on the whole table's contents (its total and,
+ * with many segments, its longest segment) and the device's compute units, not
+ * on the buffers' capacity: a request's result can differ in its rounding with
+ * the other requests of the batch.  Where it must not, use
+ * vtx_paged_decode_attention or NULL.
  */
 int vtx_paged_decode_attention_split(const uint16_t* q, uint16_t* o, const uint16_t* k_cache,
                                      const uint16_t* v_cache, int64_t cache_rows, const int32_t* kv_indptr,

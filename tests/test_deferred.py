@@ -321,6 +321,80 @@ def test_capture_hooks_only_while_carrying(carry_launches):
         _deferred.set_fusion()
 
 
+# --------------------------------------------- scratch memory and captures
+@pytest.fixture
+def captures(monkeypatch):
+    """A stand-in for torch.cuda.CUDAGraph, its current capture in state["id"]."""
+    state = {"id": 0}
+
+    class Graph:
+        def capture_begin(self):
+            state["id"] = 7
+
+        def capture_end(self):
+            state["id"] = 0
+
+    uses = _deferred._hook_uses
+    _deferred._use_capture_hooks(frozenset())
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", Graph)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: 0)
+    monkeypatch.setattr(_deferred, "_capture_of", lambda stream: state["id"])
+    yield state, Graph
+    _deferred._use_capture_hooks(frozenset())
+    monkeypatch.undo()
+    _deferred._use_capture_hooks(uses)
+
+
+def test_scratch_only_where_it_lasts(captures):
+    """Attention's scratch: outside captures and in those that torch begins, not
+    in others, whose graph would go on using memory that torch hands on."""
+    state, Graph = captures
+    own = Graph.capture_begin, Graph.capture_end
+    cpu = torch.device("cpu")
+    assert _hip._scratch(0, cpu, 0) is None
+    state["id"] = 3  # begun before any call, and by whom is not known
+    assert _hip._scratch(16, cpu, 0) is None and Graph.capture_begin is own[0]
+    state["id"] = 0
+    assert _hip._scratch(16, cpu, 0).numel() == 16
+    assert Graph.capture_begin is not own[0]  # noted from here on
+    graph = Graph()
+    graph.capture_begin()
+    assert _hip._scratch(16, cpu, 0) is not None
+    state["id"] = 8  # another stream's, begun by other means
+    assert _hip._scratch(16, cpu, 0) is None
+    state["id"] = 7
+    graph.capture_end()
+    state["id"] = 7  # (ids are not used again; a stale one would not count)
+    assert _hip._scratch(16, cpu, 0) is None
+    _deferred._use_capture_hooks(frozenset())
+    assert (Graph.capture_begin, Graph.capture_end) == own
+
+
+def test_capture_hooks_of_both_uses(captures):
+    """Noting torch's captures and launching the carry come and go apart."""
+    state, Graph = captures
+    _hip._scratch(16, torch.device("cpu"), 0)
+    noting = Graph.capture_begin
+    assert not _deferred.capture_hooks_installed()
+    _deferred._install_capture_hooks()
+    assert _deferred.capture_hooks_installed() and Graph.capture_begin is not noting
+    graph = Graph()
+    graph.capture_begin()
+    assert _hip._scratch(16, torch.device("cpu"), 0) is not None
+    _deferred.remove_capture_hooks()
+    assert Graph.capture_begin is noting and not _deferred.capture_hooks_installed()
+    assert _hip._scratch(16, torch.device("cpu"), 0) is not None
+    graph.capture_end()
+
+
+def test_no_memory_for_scratch_is_no_error(captures, monkeypatch):
+    def full(*a, **k):
+        raise torch.OutOfMemoryError("full")
+
+    monkeypatch.setattr(torch, "empty", full)
+    assert _hip._scratch(16, torch.device("cpu"), 0) is None
+
+
 def test_set_fusion_overrides_environment(monkeypatch):
     monkeypatch.setenv("VORTEX_FUSE", "1")
     monkeypatch.setenv("VORTEX_FUSE_CMEAN", "1")

@@ -202,7 +202,7 @@ def current_scope() -> Optional[Scope]:
 # layer's carry then lands at the end of the graph).  These two hooks are
 # installed with the first carry and removed by remove_capture_hooks() or by
 # switching the carry off (set_fusion(carry_cmean=False)); a process that
-# never carries keeps torch's own methods.  A carry found on a stream whose
+# never carries does without.  A carry found on a stream whose
 # capture state has changed by other means (a capture begun or ended outside
 # these two methods) is an error, raised instead of launching the mean
 # outside the work it belongs to; the carry then stays recorded
@@ -226,7 +226,7 @@ def _stream_of(dev: torch.device):
 
 
 def _capture_of(stream) -> int:
-    """Id of the graph capture `stream` takes part in (0: none)."""
+    """Id of the graph capture `stream` (or its handle) takes part in (0: none)."""
     if stream is None:
         return 0
     from . import _hip
@@ -501,51 +501,96 @@ def _install_launch_hook() -> None:
     _hip.set_pre_launch_hook(flush_carry)
 
 
-_hooked = None  # (CUDAGraph class, original capture_begin, original capture_end) while the hooks are in
+# Wrappers around torch.cuda.CUDAGraph.capture_begin / capture_end, for two
+# uses: "carry" (launch the carry first, see "Graph capture" above) and
+# "captures" (note the captures that torch begins, see scratch_lasts).  Each
+# set of uses has its own pair of wrappers; with no use left torch's own
+# methods are back.
+_hooked = None  # (CUDAGraph class, original capture_begin, original capture_end) while any wrapper is in
+_hook_uses: frozenset = frozenset()
+_hook_methods: dict = {}
+_torch_captures: set = set()  # ids of the captures in progress that torch began
+
+
+def _wrappers(uses: frozenset, begin, end):
+    import functools
+
+    def current_capture():
+        return _capture_of(torch.cuda.current_stream())
+
+    @functools.wraps(begin)
+    def capture_begin(self, *args, **kwargs):
+        if "carry" in uses:
+            flush_carry()
+        result = begin(self, *args, **kwargs)
+        if "captures" in uses:
+            _torch_captures.add(current_capture())
+        return result
+
+    @functools.wraps(end)
+    def capture_end(self, *args, **kwargs):
+        if "carry" in uses:
+            flush_carry()
+        if "captures" in uses:
+            _torch_captures.discard(current_capture())
+        return end(self, *args, **kwargs)
+
+    return capture_begin, capture_end
+
+
+def _use_capture_hooks(uses: frozenset) -> None:
+    global _hooked, _hook_uses
+    graph = getattr(torch.cuda, "CUDAGraph", None)
+    if graph is None or uses == _hook_uses:
+        return
+    if _hooked is None:
+        _hooked = (graph, graph.capture_begin, graph.capture_end)
+        _hook_methods.clear()
+    graph, begin, end = _hooked
+    if not uses:
+        graph.capture_begin, graph.capture_end = begin, end
+        _hooked = None
+    else:
+        if uses not in _hook_methods:
+            _hook_methods[uses] = _wrappers(uses, begin, end)
+        graph.capture_begin, graph.capture_end = _hook_methods[uses]
+    _hook_uses = uses
 
 
 def _install_capture_hooks() -> None:
     """Makes torch.cuda.CUDAGraph.capture_begin / capture_end launch the carry
     first (see "Graph capture" above).  Installed when a mean is first
     carried, so a process that never carries one (VORTEX_FUSE_CMEAN=0,
-    set_fusion(carry_cmean=False) or no forward_cache) keeps torch's own
-    methods; remove_capture_hooks() puts those back."""
-    global _hooked
-    import functools
-
-    graph = getattr(torch.cuda, "CUDAGraph", None)
-    if graph is None or _hooked is not None:
-        return
-    begin, end = graph.capture_begin, graph.capture_end
-
-    @functools.wraps(begin)
-    def capture_begin(self, *args, **kwargs):
-        flush_carry()
-        return begin(self, *args, **kwargs)
-
-    @functools.wraps(end)
-    def capture_end(self, *args, **kwargs):
-        flush_carry()
-        return end(self, *args, **kwargs)
-
-    graph.capture_begin, graph.capture_end = capture_begin, capture_end
-    _hooked = (graph, begin, end)
+    set_fusion(carry_cmean=False) or no forward_cache) does without;
+    remove_capture_hooks() takes this out again."""
+    _use_capture_hooks(_hook_uses | {"carry"})
 
 
 def remove_capture_hooks() -> None:
-    """Restores torch.cuda.CUDAGraph's own capture_begin / capture_end (a
-    pending carry is launched first)."""
-    global _hooked
-    if _hooked is None:
+    """Takes the carry's part out of torch.cuda.CUDAGraph's capture_begin /
+    capture_end (a pending carry is launched first)."""
+    if not capture_hooks_installed():
         return
     flush_carry()
-    graph, begin, end = _hooked
-    graph.capture_begin, graph.capture_end = begin, end
-    _hooked = None
+    _use_capture_hooks(_hook_uses - {"carry"})
 
 
 def capture_hooks_installed() -> bool:
-    return _hooked is not None
+    return "carry" in _hook_uses
+
+
+def scratch_lasts(stream: int) -> bool:
+    """Whether memory that torch allocates now, with the stream of this handle
+    current, lasts as long as the launches on it: outside any capture (the
+    stream's order), and in one that torch.cuda.CUDAGraph began (the graph's
+    own pool).  In a capture begun by other means torch would hand the memory
+    to others while the graph still uses it.  Captures are told apart from the
+    first call outside any on: one that began before counts as begun by others."""
+    capture = _capture_of(stream)
+    if capture == 0:
+        _use_capture_hooks(_hook_uses | {"captures"})
+        return True
+    return capture in _torch_captures
 
 
 _install_launch_hook()

@@ -2,8 +2,9 @@
 
 Every wrapper validates dtypes, devices, contiguity and sizes of its torch
 tensors, then launches on torch's current HIP stream of the tensors' device.
-Nothing here synchronises, reads device memory or allocates, so the wrappers
-can be recorded into a HIP graph (``torch.cuda.graph``).
+No kernel wrapper synchronises or reads device memory, and none but
+``paged_decode_attention`` allocates (scratch, where that lasts: see there), so
+they can be recorded into a HIP graph (``torch.cuda.graph``).
 
 There is no CPU fallback: a tensor that is not on a GPU, or a missing
 library, raises ``RuntimeError``.
@@ -257,10 +258,11 @@ def _stream(dev: torch.device) -> int:
 
 def stream_capture_id(stream) -> int:
     """0 if the torch stream `stream` is not being captured into a graph, else
-    an id of the capture in progress (host-side query, no launch)."""
+    an id of the capture in progress (host-side query, no launch).  stream: a
+    torch stream or its handle."""
     lib = load_library()
     out = ctypes.c_ulonglong(0)
-    _check(lib.vtx_stream_capture_id(stream.cuda_stream, ctypes.byref(out)), "stream_capture_id")
+    _check(lib.vtx_stream_capture_id(getattr(stream, "cuda_stream", stream), ctypes.byref(out)), "stream_capture_id")
     return int(out.value)
 
 
@@ -1018,11 +1020,28 @@ def set_kv_buffer(k_cache, v_cache, new_k, new_v, loc, page_size: int) -> None:
     _check(rc, "set_kv_buffer")
 
 
+def _scratch(floats: int, dev: torch.device, stream: int):
+    """fp32 scratch for launches on `stream`, the current one of `dev`, or None
+    where the call does without: inside a capture that torch did not begin (the
+    memory would be others' while the graph still uses it), or with no memory
+    left (a call that is given its output needs none)."""
+    from . import _deferred
+
+    if floats <= 0 or not _deferred.scratch_lasts(stream):
+        return None
+    try:
+        return torch.empty(floats, dtype=torch.float32, device=dev)
+    except torch.OutOfMemoryError:
+        return None
+
+
 @_plain_args
 def paged_decode_attention(q, o, k_cache, v_cache, kv_indptr, kv_indices, kv_last_page_len, batch_size: int,
                            num_kv_heads: int, sm_scale: float) -> None:
     """o[s*G + g] = softmax(sm_scale * q K^T) V over segment s's pages of the
-    block table; q / o [B*H*G, D] (or [B, H*G, D]) bf16, pools [rows, P, D]."""
+    block table; q / o [B*H*G, D] (or [B, H*G, D]) bf16, pools [rows, P, D].
+    Long segments are split over workgroups, whose partial results need scratch
+    from torch's allocator; without (see _scratch) no segment is split."""
     lib = load_library()
     dev = _require_gpu(q, o, k_cache, v_cache, kv_indptr, kv_indices, kv_last_page_len)
     for t, n in ((q, "q"), (o, "o"), (k_cache, "k_cache"), (v_cache, "v_cache")):
@@ -1039,13 +1058,12 @@ def paged_decode_attention(q, o, k_cache, v_cache, kv_indptr, kv_indices, kv_las
     if kv_indptr.numel() < B * H + 1 or kv_last_page_len.numel() < B * H:
         raise RuntimeError(f"vortex_torch: kv_indptr needs {B * H + 1} and kv_last_page_len {B * H} entries")
     with _on_device(dev):
-        n = lib.vtx_paged_decode_attention_workspace_len(B, H, G, D, P, kv_indices.numel())
-        # the chunks' partial results, on the current stream (which both launches run on)
-        ws = torch.empty(n, dtype=torch.float32, device=dev) if n > 0 else None
+        stream = _stream(dev)
+        ws = _scratch(lib.vtx_paged_decode_attention_workspace_len(B, H, G, D, P, kv_indices.numel()), dev, stream)
         rc = lib.vtx_paged_decode_attention_split(
             q.data_ptr(), o.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), rows, kv_indptr.data_ptr(),
             kv_indices.data_ptr(), kv_indices.numel(), kv_last_page_len.data_ptr(), B, H, G, D, P, float(sm_scale),
-            None if ws is None else ws.data_ptr(), n, _stream(dev))
+            None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), stream)
     _check(rc, "paged_decode_attention")
 
 
