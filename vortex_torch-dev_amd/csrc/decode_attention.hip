@@ -76,12 +76,19 @@ constexpr int kFewChunkTokens = 256;
 struct Chunks {
   uint32_t count, pages;
 };
-__device__ __forceinline__ Chunks chunks_of(const AttnArgs& a, uint32_t m, uint32_t longest, int32_t first,
-                                            int32_t end) {
-  const long long all = (long long)end - first;
+// The table's total page count, or 0 where its average is too short to split:
+// every thread of both kernels asks this first, of two loads that arrive with
+// the segment's own, so that a workgroup of a table that is not split (a short
+// one in a large buffer, whose chunks' workgroups are launched all the same)
+// does not look for the longest segment.
+__device__ __forceinline__ uint32_t split_pages(const AttnArgs& a) {
+  const long long all = (long long)a.indptr[a.segments] - a.indptr[0];
   const uint32_t total = all < 0 ? 0u : (uint32_t)(all < a.indices_len ? all : a.indices_len);
+  return (unsigned long long)total * a.P < (unsigned long long)a.min_avg_tokens * a.segments ? 0u : total;
+}
+__device__ __forceinline__ Chunks chunks_of(const AttnArgs& a, uint32_t m, uint32_t longest, uint32_t total) {
   Chunks c{1u, m};
-  if (m == 0 || (unsigned long long)total * a.P < (unsigned long long)a.min_avg_tokens * a.segments) return c;
+  if (m == 0 || total == 0) return c;
   if (a.ragged_only && 10ull * longest * a.segments <= 13ull * total) return c;
   const uint32_t least = (kMinChunkTokens + a.P - 1) / a.P, few = (kFewChunkTokens + a.P - 1) / a.P;
   uint32_t per = total / a.cus;
@@ -139,9 +146,9 @@ __device__ __forceinline__ bool attn_span(const AttnArgs& a, uint32_t* red, Span
     const long long t = (sp.pages - 1) * P + last;
     sp.tokens = t < (1LL << 30) ? (int)t : 0;  // (token indices, with the prefetch past the end, fit an int)
     if constexpr (kSplit) {
-      if (sp.tokens > 0) {
-        const Chunks c =
-            chunks_of(a, (uint32_t)sp.pages, longest_segment<T>(a, red), a.indptr[0], a.indptr[a.segments]);
+      const uint32_t total = split_pages(a);
+      if (sp.tokens > 0 && total > 0) {  // uniform
+        const Chunks c = chunks_of(a, (uint32_t)sp.pages, longest_segment<T>(a, red), total);
         sp.chunks = (int)c.count;
         if (sp.chunk < sp.chunks) {  // this chunk's pages as a segment of their own
           const int p0 = sp.chunk * (int)c.pages;
@@ -695,9 +702,10 @@ __global__ __launch_bounds__(kCombineWaves * vtx::kWave) void attention_combine_
   const int32_t last = a.last_len[seg];
   if (!(m > 0 && start >= 0 && start + m <= a.indices_len && a.rows > 0)) return;  // uniform, as the returns below
   const long long tok = (m - 1) * a.P + (last < 0 ? 0 : (last > a.P ? a.P : last));
-  if (tok <= 0 || tok >= (1LL << 30)) return;
+  const uint32_t total = split_pages(a);
+  if (tok <= 0 || tok >= (1LL << 30) || total == 0) return;
   const uint32_t longest = longest_segment<kCombineWaves * vtx::kWave>(a, s_red);
-  const int all = (int)chunks_of(a, (uint32_t)m, longest, a.indptr[0], a.indptr[a.segments]).count;
+  const int all = (int)chunks_of(a, (uint32_t)m, longest, total).count;
   if (all <= 1) return;  // written by its workgroup
   // this wave's chunks (none: wave 0's first again, with weight 0)
   const int n = all > wave ? (all - wave + kCombineWaves - 1) / kCombineWaves : 0;
@@ -809,6 +817,13 @@ struct SplitPlan {
 // 109), and one of equal lengths only pays for the combine launch (128 of 2048:
 // 32.3 us, 34.2 with it; 240 of 2048, 1 head: 42.4 and 44.5, D 64 24.3 and 26.7),
 // so the line lies where that is a few percent.
+//
+// The host knows the buffer's capacity, the kernels its contents: a short table in
+// a large buffer (32k tokens per segment) pays for the chunks' workgroups, which
+// leave at once, and for the second launch.  Two heads of 128 columns, alone / in
+// such a buffer: 8 to 128 segments of 64 tokens 5.6 to 5.8 / 7.1 to 7.6 us, of 512
+// 11.3 to 11.7 / 12.3 to 13.1; 256 of 64 6.3 / 8.7, 512 of 256 13.9 / 15.9, 1000 of
+// 256 22.9 / 26.2 and of 1024 60.5 / 60.6.
 SplitPlan split_plan(long long segments, long long indices_len, int32_t page_size, int32_t group_size,
                      int32_t head_dim) {
   const int cus = vtx::device_cu_count();
