@@ -152,6 +152,7 @@ DECODE_CONFIGS = {
 def fused_kernel_name(batch: W.DecodeBatch) -> str:
     """Kernel instance the fused launch selects (VTX_FUSED_AUTO: the library's
     split_pays and segment_threads)."""
+    from vortex_torch import _hip
     from vortex_torch._deferred import fused_layout
 
     lpr, vpl = {64: (8, 1), 128: (16, 1), 256: (16, 2), 512: (16, 4), 576: (8, 9)}[batch.head_dim]
@@ -159,9 +160,9 @@ def fused_kernel_name(batch: W.DecodeBatch) -> str:
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     layout = fused_layout()
     mp = batch.max_pages_per_request
-    auto = segments < 2 * cus if batch.head_dim >= 256 else mp > 512 and (
-        3 * segments < 2 * cus or (batch.head_dim == 128 and batch.topk <= 64 and segments * -(-mp // 256) <= 4 * cus
-                                   and (segments > cus or batch.topk > 32)))
+    lib = _hip.load_library()  # (the topK op's workspace has the staging zone)
+    auto = lib.vtx_indexer_fused_auto_layout(segments, batch.topk, batch.bos, batch.eos, mp, batch.head_dim,
+                                             lib.vtx_indexer_fused_workspace_len(segments), cus) == _hip.FUSED_SPLIT
     if layout == 2 or (layout == 0 and auto):
         # the library's split_threads / split_pass / chunk choice, with the
         # topK op's workspace (staging zone present)

@@ -216,9 +216,10 @@ int vtx_topk_select(const uint16_t* score, int64_t score_len,
  * (with the counters given, split where few segments would leave compute units
  * idle for longer than a split segment's hand-off takes: head_dim >= 256 and
  * fewer than two segments per compute unit, or head_dim <= 128, over 512 pages
- * and fewer than two for three units, or head_dim 128, over 512 pages, small
- * chunks that fit the device at once and more than one segment per unit or
- * 32 kept pages), VTX_FUSED_SEGMENT or VTX_FUSED_SPLIT.  Outputs are
+ * and fewer than two for three units, or head_dim 128, over 512 pages, the
+ * staging zone given, small chunks that fit the device at once and more than
+ * one segment per unit or 32 kept pages), VTX_FUSED_SEGMENT or
+ * VTX_FUSED_SPLIT.  Outputs are
  * identical in every mode.
  *
  * schedule (optional, NULL for none): the fused_schedule vtx_plan_decode
@@ -243,6 +244,16 @@ int vtx_indexer_fused(const uint16_t* q, int64_t q_rows, int32_t group_size,
  * count.  Allocate it zeroed once and pass it to every call.
  */
 int64_t vtx_indexer_fused_workspace_len(int32_t segments);
+
+/*
+ * The layout that VTX_FUSED_AUTO takes (VTX_FUSED_SEGMENT or VTX_FUSED_SPLIT)
+ * on a device of that many compute units with a workspace of seg_counters_len
+ * entries (0: none); a negative code for bad arguments.  No launch, no device
+ * needed.
+ */
+int vtx_indexer_fused_auto_layout(int32_t eff_batch_size, int32_t topk_val, int32_t reserved_bos,
+                                  int32_t reserved_eos, int32_t max_num_pages, int32_t head_dim,
+                                  int64_t seg_counters_len, int32_t compute_units);
 
 /*
  * vtx_indexer_fused without the seg_counters workspace: the split layout's

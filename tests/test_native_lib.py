@@ -80,6 +80,31 @@ def test_page_reduce_sharing_leaves_no_wave_a_queue(cols, types):
                     assert share.value == 16, what
 
 
+@pytest.mark.parametrize("segments", [1, 170, 171, 200, 256, 257, 304, 341, 342, 511, 512, 600])
+@pytest.mark.parametrize("dim", [64, 128, 256, 576])
+def test_auto_layout_needs_the_staging_zone_for_four_wave_chunks(segments, dim):
+    """On 256 compute units: the four-wave chunks that let AUTO split past two
+    segments for three units exist only with the staging zone, so a workspace
+    of counters alone, or none, never splits there."""
+    lib = _hip.load_library()
+    full = lib.vtx_indexer_fused_workspace_len(segments)
+    for pages in (16, 512, 513, 600, 1024, 2046, 8192):
+        for topk in (16, 32, 33, 64, 65):
+            def split(entries):
+                rc = lib.vtx_indexer_fused_auto_layout(segments, topk, 1, 1, pages, dim, entries, 256)
+                assert rc in (_hip.FUSED_SEGMENT, _hip.FUSED_SPLIT)
+                return rc == _hip.FUSED_SPLIT
+            what = (segments, pages, topk, dim)
+            idle = segments < 512 if dim >= 256 else pages > 512 and 3 * segments < 512
+            chunks = -(-(pages - 2) // 256)
+            quad = (dim == 128 and pages > 512 and topk <= 64 and chunks <= 16 and segments <= 512
+                    and segments * chunks <= 1024 and (segments > 256 or topk > 32))
+            assert split(full) == (idle or quad), what
+            assert split(segments) == idle, what
+            assert not split(segments - 1) and not split(0), what
+    assert lib.vtx_indexer_fused_auto_layout(4, 30, 1, 1, 512, 100, 0, 256) == -1
+
+
 def test_missing_library_fails_loudly(tmp_path):
     with pytest.raises(RuntimeError, match="not found"):
         _hip.load_library(tmp_path / "nope.so")

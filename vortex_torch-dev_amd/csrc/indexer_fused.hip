@@ -1261,13 +1261,30 @@ int split_chunk(int dim, bool large, bool quad) {
 // longer fit, 26.9 / 31.3), and with more than 32 kept pages, whose select
 // takes a 16-wave workgroup longer (208 of 600, top-64 17.2 / 16.4, top-30 15.2
 // / 16.3; 208 of 1500, which do not fit, 26.7 / 32.1).
-bool split_pays(long long segments, long long max_pages, int dim, int topk, int cus) {
+//
+// quad: those small chunks of four waves, which need the staging zone.  With a
+// workspace of counters alone the chunks are 8-wave ones that hand over without
+// it and always lose there (top-64, segment / counters / zone: 208 of 520 equal
+// pages 11.8 / 16.4 / 11.3, 304 of 520 16.3 / 18.3 / 13.2, of 768 19.0 / 22.1 /
+// 16.4).
+bool split_pays(long long segments, long long max_pages, int dim, int topk, bool quad, int cus) {
   if (dim >= 256) return segments < 2LL * cus;
   if (max_pages <= 512) return false;
-  const long long chunk = split_chunk(dim, false, true);
-  const bool fits = dim == 128 && topk <= vtx::kMaxBitonicRunK && segments <= kStageMaxSegments &&
-                    segments * ((max_pages + chunk - 1) / chunk) <= 4LL * cus;
-  return 3 * segments < 2LL * cus || (fits && (segments > cus || topk > 32));
+  return 3 * segments < 2LL * cus || (quad && (segments > cus || topk > 32));
+}
+
+long long middle_pages(long long max_pages, int bos, int eos) {
+  return max_pages - bos - eos > 1 ? max_pages - bos - eos : 1;
+}
+
+// Four-wave workgroups for the small chunks: at D = 128 when every chunk of
+// every segment is one workgroup's (all on the chip at once) and the chunks
+// stage their lists.
+bool quad_chunks(long long segments, long long middle, int dim, int topk, bool zone, int cus) {
+  const long long small = split_chunk(dim, false, true);
+  const long long chunks = (middle + small - 1) / small;
+  return dim == 128 && zone && topk <= vtx::kMaxBitonicRunK && segments <= kStageMaxSegments &&
+         chunks <= kStageLists && segments * chunks <= (1024LL / 256) * cus;
 }
 
 // blocks: the grid, xcd: work ids per XCD (8 * xcd workgroups take work
@@ -1336,6 +1353,24 @@ extern "C" int vtx_indexer_fused_supported(int32_t head_dim) {
 
 extern "C" int64_t vtx_indexer_fused_workspace_len(int32_t segments) {
   return segments < 0 ? -1 : (int64_t)segments + kStageZoneInts;
+}
+
+extern "C" int vtx_indexer_fused_auto_layout(int32_t eff_batch_size, int32_t topk_val, int32_t reserved_bos,
+                                             int32_t reserved_eos, int32_t max_num_pages, int32_t head_dim,
+                                             int64_t seg_counters_len, int32_t compute_units) {
+  vtx::clear_error();
+  if (eff_batch_size < 0 || reserved_bos < 0 || reserved_eos < 0 || seg_counters_len < 0 || compute_units < 1 ||
+      !vtx_indexer_fused_supported(head_dim))
+    return vtx::fail(VTX_E_INVALID, "indexer_fused_auto_layout: bad arguments");
+  const bool zone = seg_counters_len >= kStageZoneInts;
+  const long long pages = max_num_pages > 0 ? max_num_pages : 0;
+  const int topk = topk_val > 0 ? topk_val : 0;
+  const bool quad = quad_chunks(eff_batch_size, middle_pages(pages, reserved_bos, reserved_eos), head_dim, topk, zone,
+                                compute_units);
+  return seg_counters_len - (zone ? kStageZoneInts : 0) >= eff_batch_size &&
+                 split_pays(eff_batch_size, pages, head_dim, topk, quad, compute_units)
+             ? VTX_FUSED_SPLIT
+             : VTX_FUSED_SEGMENT;
 }
 
 namespace {
@@ -1475,8 +1510,10 @@ int fused_impl(const uint16_t* q, int64_t q_rows, int32_t group_size, const uint
   const int cus = vtx::device_cu_count();
   if (cus <= 0) return vtx::fail(VTX_E_DEVICE, "indexer_fused: cannot query the compute unit count");
 
-  const bool split = mode == VTX_FUSED_SPLIT ||
-                     (mode == VTX_FUSED_AUTO && have_counters && split_pays(eff_batch_size, want, head_dim, a.topk, cus));
+  const long long mid = middle_pages(want, reserved_bos, reserved_eos);
+  const bool quad = quad_chunks(eff_batch_size, mid, head_dim, a.topk, zone != nullptr, cus);
+  const bool split = mode == VTX_FUSED_SPLIT || (mode == VTX_FUSED_AUTO && have_counters &&
+                                                 split_pays(eff_batch_size, want, head_dim, a.topk, quad, cus));
   // The CMean runs inside the launch for decode-sized loc and a 16-byte
   // aligned K pool: in the segment layout for rows of one 16-byte vector per
   // lane (its tile layout is then the scoring layout), in the split layout
@@ -1513,15 +1550,9 @@ int fused_impl(const uint16_t* q, int64_t q_rows, int32_t group_size, const uint
     // (its query mean of up to 16 heads, its staged list, its count-in) then
     // serves twice the pages, and a segment hands over half as many lists
     // (C5: 13.7 -> 12.8 us per launch; at C3 the large chunks are slower).
-    const long long mid = want - reserved_bos - reserved_eos > 1 ? want - reserved_bos - reserved_eos : 1;
     // (split workgroups resident at once: 16 waves per CU)
     const long long small = split_chunk(head_dim, false, false);
     const long long small_chunks = (mid + small - 1) / small;
-    // four-wave workgroups at D = 128 when every chunk of every segment is
-    // one workgroup's and the chunks stage their lists
-    const bool quad = head_dim == 128 && zone != nullptr && a.topk <= vtx::kMaxBitonicRunK &&
-                      eff_batch_size <= kStageMaxSegments && small_chunks <= kStageLists &&
-                      (long long)eff_batch_size * small_chunks <= (1024LL / 256) * cus;
     const bool large = head_dim >= 512 ||
                        (long long)eff_batch_size * small_chunks > (1024LL / split_threads(head_dim, false, quad)) * cus;
     const long long resident = (1024LL / split_threads(head_dim, large, quad)) * cus;

@@ -71,6 +71,7 @@ _SIGNATURES = {
         ctypes.c_int,
     ),
     "vtx_indexer_fused_workspace_len": ([_i32], ctypes.c_int64),
+    "vtx_indexer_fused_auto_layout": ([_i32, _i32, _i32, _i32, _i32, _i32, _i64, _i32], ctypes.c_int),
     "vtx_indexer_fused_noalloc_reset": ([_vp], ctypes.c_int),
     "vtx_indexer_fused_supported": ([_i32], ctypes.c_int),
     "vtx_indexer_fused_cmean": (
