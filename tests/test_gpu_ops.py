@@ -740,8 +740,9 @@ def test_decode_attention_head_shapes(gpu, D, G):
 
 @pytest.mark.parametrize("G", [1, 2, 4])
 def test_decode_attention_long_segment(gpu, G):
-    """Segments of more pages than the kernel stages in LDS (2048) read their
-    page rows from the table; a short and an empty request beside them."""
+    """Segments of more pages than the kernel stages in LDS (2048), cut into
+    chunks that are staged (whole ones: below); a short and an empty request
+    beside them."""
     from vortex_torch.decode_attention import dense_decode_attention
     from vortex_torch.indexer.utils_sglang import plan_decode
 
@@ -911,3 +912,108 @@ def test_decode_attention_ignores_rows_of_others(gpu, G, D, P, lens, outside):
     for o in (paged_decode_attention(q, k, v, ip, idx, last, len(lens), 1),
               _attend_whole(q, k, v, ip, idx, last, len(lens), G, D, P)):
         np.testing.assert_allclose(_f(_bits(o)), exp, rtol=2 ** -7, atol=1e-4)
+
+
+def _split_call(q, o, k, v, ip, idx, last, S, G, D, P, ws, floats):
+    return _hip.load_library().vtx_paged_decode_attention_split(
+        q.data_ptr(), o.data_ptr(), k.data_ptr(), v.data_ptr(), k.shape[0], ip.data_ptr(), idx.data_ptr(),
+        idx.numel(), last.data_ptr(), S, 1, G, D, P, 1.0 / np.sqrt(D), ws, floats,
+        torch.cuda.current_stream().cuda_stream)
+
+
+def _attend_f64(q, k, v, ip, idx, last, G, D, P):
+    """Each segment's attention in 64 bits, [S, G, D]."""
+    ip, last = ip.tolist(), last.tolist()
+    out = torch.zeros((len(last), G, D), dtype=torch.float64, device=q.device)
+    for s in range(len(last)):
+        rows = idx[ip[s]:ip[s + 1]].long()
+        tok = (rows.numel() - 1) * P + last[s]
+        if rows.numel() and tok > 0:
+            kk = k[rows].view(-1, D)[:tok].double()
+            vv = v[rows].view(-1, D)[:tok].double()
+            w = torch.softmax(kk @ q.view(-1, G, D)[s].double().t().contiguous() / np.sqrt(D), 0)
+            out[s] = w.t().contiguous() @ vv
+    return out
+
+
+@pytest.mark.parametrize("name", sorted(_SPLIT_TABLES))
+def test_decode_attention_split_partials(gpu, name):
+    """The chunks' fp32 partial results, weighed in 64 bits, are the attention
+    in 64 bits to 1e-5 (2-norm per query head; fp32 sums, scores and weights
+    are each good to about 1e-6), the output is their bf16 rounding, whatever
+    the scratch held before, and the tables that must split do: every one but
+    that of many equal segments."""
+    lens, H, P, G, D = _SPLIT_TABLES[name]
+    lens = [n for n in lens for _ in range(H)]
+    S = len(lens)
+    rows, (ip, idx, last), _ = _hand_table(lens, P, gpu, 7)
+    k, v = W.randn_bf16((rows, P, D), 51, gpu), W.randn_bf16((rows, P, D), 52, gpu)
+    q = W.randn_bf16((S * G, D), 53, gpu)
+    floats = _hip.load_library().vtx_paged_decode_attention_workspace_len(S, 1, G, D, P, idx.numel())
+    nsplit = floats // (S * G * (D + 2))
+    assert nsplit > 1 and floats == S * nsplit * G * (D + 2)
+    unwritten = -2.0 ** 100
+    outs = []
+    for fill in (unwritten, float("nan")):
+        ws, o = torch.full((floats,), fill, device=gpu), torch.full_like(q, 7.0)
+        assert _split_call(q, o, k, v, ip, idx, last, S, G, D, P, ws.data_ptr(), floats) == 0
+        outs.append(o)
+        if fill == unwritten:
+            acc = ws[:S * nsplit * G * D].view(S, nsplit, G, D).double()
+            ml = ws[S * nsplit * G * D:].view(S, nsplit, G, 2).double()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    written = (ml[..., 0] != unwritten).all(-1)  # [S, nsplit]
+    assert torch.equal(written, (ml[..., 0] != unwritten).any(-1)) and torch.equal(written, (acc != unwritten).any(-1).any(-1))
+    chunks = written.sum(1)
+    assert torch.equal(written, torch.arange(nsplit, device=gpu)[None, :] < chunks[:, None])
+    assert not (chunks == 1).any()  # a whole segment writes its result
+    if name == "equal":
+        assert int(chunks.sum()) == 0
+        return
+    assert int(chunks[int(np.argmax(lens))]) > 1
+    M = ml[..., 0].masked_fill(~written[..., None], float("-inf"))
+    f = torch.exp(M - M.amax(1, keepdim=True)).masked_fill(~written[..., None], 0.0)
+    split = chunks > 0
+    combined = (f[..., None] * acc).sum(1)[split] / (f * ml[..., 1]).sum(1)[split][..., None]
+    exp = _attend_f64(q, k, v, ip, idx, last, G, D, P)[split]
+    err = (combined - exp).norm(dim=-1) / exp.norm(dim=-1)
+    assert float(err.max()) < 1e-5
+    got = outs[0].view(S, G, D)[split].double()
+    rms = combined.pow(2).mean().sqrt()
+    assert bool(((got - combined).abs() <= combined.abs() * (2.0 ** -8 + 1e-5) + 1e-5 * rms).all())
+
+
+def test_decode_attention_split_refuses_a_bad_workspace(gpu):
+    """Too short or misaligned is an error before any launch; none splits nothing."""
+    lens, G, D, P = [3000, 2000], 2, 128, 16
+    rows, (ip, idx, last), _ = _hand_table(lens, P, gpu, 9)
+    k, v = W.randn_bf16((rows, P, D), 51, gpu), W.randn_bf16((rows, P, D), 52, gpu)
+    q = W.randn_bf16((2 * G, D), 53, gpu)
+    lib = _hip.load_library()
+    floats = lib.vtx_paged_decode_attention_workspace_len(2, 1, G, D, P, idx.numel())
+    ws, o = torch.zeros(floats + 4, device=gpu), torch.full_like(q, 7.0)
+    for ptr, n in ((ws.data_ptr(), floats - 1), (ws.data_ptr() + 4, floats), (ws.data_ptr(), 0)):
+        assert _split_call(q, o, k, v, ip, idx, last, 2, G, D, P, ptr, n) == -1
+        assert b"workspace" in lib.vtx_last_error()
+    torch.cuda.synchronize()
+    assert bool((o == 7.0).all()) and bool((ws == 0).all())
+    assert _split_call(q, o, k, v, ip, idx, last, 2, G, D, P, None, 0) == 0
+    assert torch.equal(o, _attend_whole(q, k, v, ip, idx, last, 2, G, D, P))
+
+
+@pytest.mark.parametrize("G,D,P", [(1, 64, 16), (2, 128, 16), (2, 256, 16), (4, 128, 16), (8, 64, 16), (4, 128, 8)])
+def test_decode_attention_whole_segment_past_the_staged_pages(gpu, G, D, P):
+    """A whole segment of more pages than are staged in LDS (2048) reads its page
+    rows from the table, in both kernels: to 1e-5 of the attention in 64 bits
+    before the bf16 rounding; entries outside the pool and rows of nobody that
+    are NaN leave no trace."""
+    lens = [2049 * P + 5, 2048 * P, 37, 2300 * P - 1]
+    rows, (ip, idx, last), kept = _hand_table(lens, P, gpu, 11, outside=True)
+    k, v = W.randn_bf16((rows, P, D), 61, gpu), W.randn_bf16((rows, P, D), 62, gpu)
+    q = W.randn_bf16((len(lens) * G, D), 63, gpu)
+    kip, kidx, klast = (torch.as_tensor(t, device=gpu) for t in kept)
+    exp = _attend_f64(q, k, v, kip, kidx, klast, G, D, P)
+    k[0], v[0] = float("nan"), float("nan")
+    o = _attend_whole(q, k, v, ip, idx, last, len(lens), G, D, P).view(len(lens), G, D).double()
+    rms = exp.pow(2).mean(-1, keepdim=True).sqrt()
+    assert bool(((o - exp).abs() <= exp.abs() * (2.0 ** -8 + 1e-5) + 1e-5 * rms).all())
