@@ -65,9 +65,9 @@ constexpr int kFewChunkTokens = 256;
 //
 // A table is split when its segments hold min_avg_tokens on average and,
 // with half a segment per CU and more, the longest is over 1.3 times the
-// average (split_plan says why).  A workgroup takes about 5.5 us + 12.6 us per
-// 1024 tokens (its dot products, not its loads, set that; 1024 threads took as
-// long) until all of them together reach the card's read rate, the combine
+// average (split_plan says why).  A workgroup takes about 5.5 us + 14 us per
+// 1024 tokens (two heads of 128 columns: its dot products, not its loads, set
+// that; 1024 threads took as long) until all of them together reach the card's read rate, the combine
 // launch 2.5 us.  So a few short segments want one chunk of 128-256 tokens per
 // CU (8 segments of 2048 tokens: 11.4 us with chunks of 128, 13.1 with 256; 64
 // segments of 1024: 19.0 and 16.0), and long ones four chunks per CU in all,

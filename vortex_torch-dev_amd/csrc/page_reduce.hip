@@ -253,7 +253,7 @@ struct Sharing {
 // whose pages all close together (256 tiles per head and block) find waves:
 // they cost nothing where there is no work.  CMax + CMin (every statistic
 // accumulated, one tile per wave), 16-token pages of 128 columns, 8 heads: 32
-// blocks 42 us with 8 workgroups each, 36 with 16; 512 blocks, read from
+// blocks 15.8 us with 8 workgroups each, 12.7 with 16; 512 blocks, read from
 // memory, 247 with one and 154 with eight; 64 columns, 2 heads, 32 blocks 42
 // with one and 7.2 with 16.  Decode of 1024 requests, one head, 256-token
 // pages that all close: 739 us with one workgroup per block, 50 with 16.
@@ -265,10 +265,10 @@ struct Sharing {
 // waves to take them one at a time: from 8192 tiles on (4096 with two
 // statistics or more, whose fold is longer), or where a block has more than
 // two rounds' (one round's) tiles.  CMean, 128 columns, one tile per wave /
-// lane tiles: 8 heads, 16 blocks 5.1 / 6.2 us, 128 blocks 15.1 / 13.1; one
-// head, 4 blocks 3.8 / 4.8, 128 blocks 4.4 / 7.1; CMean + CMax, 8 heads, 8
+// lane tiles: 8 heads, 16 blocks 5.6 / 6.8 us, 128 blocks 14.7 / 13.1; one
+// head, 4 blocks 3.8 / 4.7, 128 blocks 4.4 / 7.0; CMean + CMax, 8 heads, 8
 // blocks 6.0 / 5.3.  256 columns and more have two tiles or one per wave, which
-// a single statistic gains nothing from (8 heads, 128 blocks 25.2 / 27.9).
+// a single statistic gains nothing from (8 heads, 128 blocks 25.2 / 26.8).
 Sharing share_tiles(long long blocks, int page, int heads, int rows, bool vec, int lpr, int need) {
   const long long tiles = (page < kThreads ? kThreads / page : 1) * (long long)heads;
   const int stats = __builtin_popcount(need);
