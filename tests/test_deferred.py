@@ -335,14 +335,14 @@ def captures(monkeypatch):
             state["id"] = 0
 
     uses = _deferred._hook_uses
-    _deferred._use_capture_hooks(frozenset())
+    _deferred._use_capture_hooks(drop=uses)
     monkeypatch.setattr(torch.cuda, "CUDAGraph", Graph)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: 0)
     monkeypatch.setattr(_deferred, "_capture_of", lambda stream: state["id"])
     yield state, Graph
-    _deferred._use_capture_hooks(frozenset())
+    _deferred._use_capture_hooks(drop=_deferred._hook_uses)
     monkeypatch.undo()
-    _deferred._use_capture_hooks(uses)
+    _deferred._use_capture_hooks(add=uses)
 
 
 def test_scratch_only_where_it_lasts(captures):
@@ -366,7 +366,7 @@ def test_scratch_only_where_it_lasts(captures):
     graph.capture_end()
     state["id"] = 7  # (ids are not used again; a stale one would not count)
     assert _hip._scratch(16, cpu, 0) is None
-    _deferred._use_capture_hooks(frozenset())
+    _deferred._use_capture_hooks(drop=_deferred._hook_uses)
     assert (Graph.capture_begin, Graph.capture_end) == own
 
 
@@ -385,6 +385,27 @@ def test_capture_hooks_of_both_uses(captures):
     assert Graph.capture_begin is noting and not _deferred.capture_hooks_installed()
     assert _hip._scratch(16, torch.device("cpu"), 0) is not None
     graph.capture_end()
+
+
+def test_capture_hooks_installed_by_many_threads_wrap_once(captures):
+    import threading
+
+    state, Graph = captures
+    own = Graph.capture_begin, Graph.capture_end
+    go = threading.Barrier(8)
+
+    def use(n):
+        go.wait()
+        for _ in range(50):
+            _hip._scratch(16, torch.device("cpu"), 0)
+            (_deferred._install_capture_hooks if n % 2 else _deferred.remove_capture_hooks)()
+
+    threads = [threading.Thread(target=use, args=(n,)) for n in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert _deferred._hooked[1:] == own and Graph.capture_begin.__wrapped__ is own[0]
 
 
 def test_no_memory_for_scratch_is_no_error(captures, monkeypatch):

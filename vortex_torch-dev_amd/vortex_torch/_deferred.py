@@ -507,8 +507,10 @@ def _install_launch_hook() -> None:
 # set of uses has its own pair of wrappers; with no use left torch's own
 # methods are back.
 _hooked = None  # (CUDAGraph class, original capture_begin, original capture_end) while any wrapper is in
+_CARRY, _CAPTURES = frozenset({"carry"}), frozenset({"captures"})
 _hook_uses: frozenset = frozenset()
 _hook_methods: dict = {}
+_hook_lock = threading.RLock()
 _torch_captures: set = set()  # ids of the captures in progress that torch began
 
 
@@ -538,23 +540,27 @@ def _wrappers(uses: frozenset, begin, end):
     return capture_begin, capture_end
 
 
-def _use_capture_hooks(uses: frozenset) -> None:
+def _use_capture_hooks(add: frozenset = frozenset(), drop: frozenset = frozenset()) -> None:
     global _hooked, _hook_uses
-    graph = getattr(torch.cuda, "CUDAGraph", None)
-    if graph is None or uses == _hook_uses:
+    if add <= _hook_uses and not drop & _hook_uses:
         return
-    if _hooked is None:
-        _hooked = (graph, graph.capture_begin, graph.capture_end)
-        _hook_methods.clear()
-    graph, begin, end = _hooked
-    if not uses:
-        graph.capture_begin, graph.capture_end = begin, end
-        _hooked = None
-    else:
-        if uses not in _hook_methods:
-            _hook_methods[uses] = _wrappers(uses, begin, end)
-        graph.capture_begin, graph.capture_end = _hook_methods[uses]
-    _hook_uses = uses
+    with _hook_lock:
+        uses = (_hook_uses | add) - drop
+        graph = getattr(torch.cuda, "CUDAGraph", None)
+        if graph is None or uses == _hook_uses:
+            return
+        if _hooked is None:
+            _hooked = (graph, graph.capture_begin, graph.capture_end)
+            _hook_methods.clear()
+        graph, begin, end = _hooked
+        if not uses:
+            graph.capture_begin, graph.capture_end = begin, end
+            _hooked = None
+        else:
+            if uses not in _hook_methods:
+                _hook_methods[uses] = _wrappers(uses, begin, end)
+            graph.capture_begin, graph.capture_end = _hook_methods[uses]
+        _hook_uses = uses
 
 
 def _install_capture_hooks() -> None:
@@ -563,7 +569,7 @@ def _install_capture_hooks() -> None:
     carried, so a process that never carries one (VORTEX_FUSE_CMEAN=0,
     set_fusion(carry_cmean=False) or no forward_cache) does without;
     remove_capture_hooks() takes this out again."""
-    _use_capture_hooks(_hook_uses | {"carry"})
+    _use_capture_hooks(add=_CARRY)
 
 
 def remove_capture_hooks() -> None:
@@ -572,7 +578,7 @@ def remove_capture_hooks() -> None:
     if not capture_hooks_installed():
         return
     flush_carry()
-    _use_capture_hooks(_hook_uses - {"carry"})
+    _use_capture_hooks(drop=_CARRY)
 
 
 def capture_hooks_installed() -> bool:
@@ -588,7 +594,7 @@ def scratch_lasts(stream: int) -> bool:
     first call outside any on: one that began before counts as begun by others."""
     capture = _capture_of(stream)
     if capture == 0:
-        _use_capture_hooks(_hook_uses | {"captures"})
+        _use_capture_hooks(add=_CAPTURES)
         return True
     return capture in _torch_captures
 
